@@ -45,6 +45,7 @@ LIB_SOURCES = (
         [f"-DSEGTACO_BATCH_DT={dt}", f"-DSEGTACO_BATCH_SV={sv}"])
        for dt in range(3) for sv in range(2)]
     + [("k_eb_inst.hip", f"k_eb_{dt}", [f"-DSEGTACO_EB_DT={dt}"]) for dt in range(3)]
+    + [("k_seg.hip", f"k_seg_{dt}", [f"-DSEGTACO_SEG_DT={dt}"]) for dt in range(3)]
 )
 # rocSPARSE backs the vendor comparison row only (vendor.cpp).
 LIB_LINK = ["-L/opt/rocm/lib", "-lrocsparse", "-Wl,-rpath,/opt/rocm/lib"]

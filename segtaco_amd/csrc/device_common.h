@@ -196,6 +196,31 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// x of the lane a DPP row shift (CTRL) names; 0 where that lane lies outside
+// the row of 16 lanes.
+template <int CTRL>
+__device__ __forceinline__ int32_t dpp_or_zero(int32_t x) {
+  return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xF, 0xF, false);
+}
+
+// Inclusive scan over the wave's 64 lanes, sum (kMax false) or maximum
+// (kMax true), of values >= 0 (0 is the identity of both): shifts by 1, 2,
+// 4 and 8 lanes inside each row of 16 (DPP, no LDS), then each row adds the
+// totals of the rows below it (lanes 15, 31 and 47).
+template <bool kMax>
+__device__ __forceinline__ int32_t wave_scan(int32_t x) {
+  auto op = [](int32_t u, int32_t v) { return kMax ? max(u, v) : u + v; };
+  x = op(x, dpp_or_zero<0x111>(x));  // row_shr:1
+  x = op(x, dpp_or_zero<0x112>(x));  // row_shr:2
+  x = op(x, dpp_or_zero<0x114>(x));  // row_shr:4
+  x = op(x, dpp_or_zero<0x118>(x));  // row_shr:8
+  const int32_t b1 = __builtin_amdgcn_readlane(x, 15);
+  const int32_t b2 = op(b1, __builtin_amdgcn_readlane(x, 31));
+  const int32_t b3 = op(b2, __builtin_amdgcn_readlane(x, 47));
+  const int row = (threadIdx.x & 63) >> 4;
+  return row == 0 ? x : op(x, row == 1 ? b1 : row == 2 ? b2 : b3);
+}
+
 // V consecutive FP32 values to C (aligned to V floats; V == 8 is two float4).
 template <int V>
 __device__ __forceinline__ void store_vec(float *__restrict__ p,

@@ -13,6 +13,7 @@
 #include "bd.h"
 #include "cs.h"
 #include "launch.h"
+#include "seg.h"
 #include "spmv.h"
 
 namespace segtaco {
@@ -624,12 +625,23 @@ int32_t spmm_impl(const segtaco_csr_t *A, const void *B, int32_t b_dtype,
   a.tile_row = reinterpret_cast<int32_t *>(w + L.rows_off);
   if (prepare) prep_record(ws, nullptr);
   SEGTACO_HIP(mark(0));
+  const int64_t tiles_per_block = (int64_t)kWavesPerBlock * (64 / plan.col_lanes);
+  if (run && plan.schedule == SEGTACO_EB_SR) {
+    SegArgs g;
+    if (const int32_t sv =
+            seg_plan(b_dtype, a, ceil_div(L.ntiles, tiles_per_block) * a.panels, &g)) {
+      SEGTACO_HIP(mark(1));
+      SEGTACO_HIP(launch_seg(b_dtype, sv, g, stream));
+      SEGTACO_HIP(mark(2));
+      SEGTACO_HIP(launch_seg_fixup(g, stream));
+      SEGTACO_HIP(mark(3));
+      return SEGTACO_OK;
+    }
+  }
   SEGTACO_HIP(launch_tile_rows_fix(V, a, stream));
   SEGTACO_HIP(mark(1));
   if (!run) return SEGTACO_OK;
   if (plan.schedule == SEGTACO_EB_SR) {
-    const int64_t tiles_per_block =
-        (int64_t)kWavesPerBlock * (64 / plan.col_lanes);
     a.nblocks = (int32_t)ceil_div(L.ntiles, tiles_per_block);
     SEGTACO_HIP(launch_eb_sr(b_dtype, V, a, stream));
   } else {
