@@ -118,16 +118,15 @@ struct BChunk {
   uint4 q[kPasses];
 };
 
-// full8: B 16-byte aligned with ldb and N multiples of 8 (uniform over the
-// launch), so each thread's 8-column segment lies wholly inside or wholly
-// past N. Then every segment is one 16-byte load with no branch around it —
+// kFull8: B 16-byte aligned with ldb and N multiples of 8, so each thread's
+// 8-column segment lies wholly inside or wholly past N. Then every segment is
+// one aligned 16-byte load with no branch around it —
 // rows past the window or K read row cmin, segments past N column 0, and
 // both are replaced by zeros — so the number of loads in flight is the same
 // on every path and a wait for one chunk leaves the later chunks in flight.
-template <int CT>
+template <int CT, bool kFull8>
 __device__ __forceinline__ void bd_load_chunk(const KArgs &a, int32_t cmin, int32_t W,
-                                              int32_t k0, int32_t col0, bool full8,
-                                              BChunk<CT> &ch) {
+                                              int32_t k0, int32_t col0, BChunk<CT> &ch) {
   using C = BChunk<CT>;
   const uint16_t *B = static_cast<const uint16_t *>(a.B);
   const int tid = threadIdx.x;
@@ -137,7 +136,7 @@ __device__ __forceinline__ void bd_load_chunk(const KArgs &a, int32_t cmin, int3
     const int32_t k = k0 + tid / C::kSegs + i * C::kRowsPerPass;
     const int32_t grow = cmin + k;
     const bool row_ok = k < W && grow < a.K;
-    if (full8) {
+    if constexpr (kFull8) {
       const bool ok = row_ok && col < a.N;
       const uint16_t *src = B + (int64_t)(row_ok ? grow : cmin) * a.ldb + (col < a.N ? col : 0);
       const uint4 q = *reinterpret_cast<const uint4 *>(src);
@@ -146,11 +145,16 @@ __device__ __forceinline__ void bd_load_chunk(const KArgs &a, int32_t cmin, int3
       uint4 q = make_uint4(0u, 0u, 0u, 0u);
       if (row_ok) {
         const uint16_t *src = B + (int64_t)grow * a.ldb + col;
-        uint32_t w[4] = {0u, 0u, 0u, 0u};
+        if (col + 8 <= a.N) {
+          // whole segment: one load at element alignment
+          __builtin_memcpy(&q, __builtin_assume_aligned(src, 2), sizeof(q));
+        } else {
+          uint32_t w[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
-          if (col + u < a.N) w[u >> 1] |= (uint32_t)src[u] << (16 * (u & 1));
-        q = make_uint4(w[0], w[1], w[2], w[3]);
+          for (int u = 0; u < 8; ++u)
+            if (col + u < a.N) w[u >> 1] |= (uint32_t)src[u] << (16 * (u & 1));
+          q = make_uint4(w[0], w[1], w[2], w[3]);
+        }
       }
       ch.q[i] = q;
     }
@@ -197,7 +201,7 @@ struct BdShared {
 // and returns true, or returns false without writing when the scatter finds
 // an entry outside the window or a row whose columns do not increase.
 // Called by the whole workgroup (uniform arguments).
-template <int DT, int CT, int RB, int RT>
+template <int DT, int CT, int RB, int RT, bool kFull8>
 __device__ bool bd_mfma(const KArgs &a, BdShared<CT, RB> &sh, const int32_t *pos, int32_t r0,
                         int32_t rows, int32_t col0, int32_t cmin, int32_t cmax,
                         int32_t stride) {
@@ -205,16 +209,13 @@ __device__ bool bd_mfma(const KArgs &a, BdShared<CT, RB> &sh, const int32_t *pos
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int32_t W = cmax - cmin + 1;
   const int32_t Wk = (W + kBdKC - 1) & ~(kBdKC - 1);  // MFMA K steps of 16
-  // branch-free 16-byte B loads (bd_load_chunk)
-  const bool full8 = (reinterpret_cast<uintptr_t>(a.B) & 15) == 0 && (a.ldb & 7) == 0 &&
-                     (a.N & 7) == 0;
   uint16_t *sA = sh.A;
   __syncthreads();  // a previous pass has finished with the LDS tiles
 
   // the first B chunk and the block's entries in flight together, while the
   // A tile's window is zeroed
   BChunk<CT> ch;
-  bd_load_chunk<CT>(a, cmin, W, 0, col0, full8, ch);
+  bd_load_chunk<CT, kFull8>(a, cmin, W, 0, col0, ch);
   const int32_t pb = pos[0], n = pos[rows] - pb;
   for (int32_t i = wave; i < kBdRows * RT; i += kWavesPerBlock)
     for (int32_t w = lane; w < Wk / 2; w += 64)
@@ -292,7 +293,7 @@ __device__ bool bd_mfma(const KArgs &a, BdShared<CT, RB> &sh, const int32_t *pos
   for (int32_t k0 = 0; k0 < Wk; k0 += kBdKC) {
     __syncthreads();  // A scattered / previous chunk consumed
     bd_store_chunk<CT>(sh.B, ch);
-    if (k0 + kBdKC < Wk) bd_load_chunk<CT>(a, cmin, W, k0 + kBdKC, col0, full8, ch);
+    if (k0 + kBdKC < Wk) bd_load_chunk<CT, kFull8>(a, cmin, W, k0 + kBdKC, col0, ch);
     __syncthreads();
     v8s bv[CT];
 #pragma unroll
@@ -310,23 +311,62 @@ __device__ bool bd_mfma(const KArgs &a, BdShared<CT, RB> &sh, const int32_t *pos
   // C tiles: lane holds rows (r%4) + 4*(lane/32) + 8*(r/4), column lane%32.
   // Non-temporal stores: C (1.07 GB on the banded 1M^2 workload at N = 256)
   // is never read back here, and allocating it in L2 evicts the B-window
-  // lines neighbouring blocks reuse (5 % less FETCH, 1-3 % less time).
+  // lines neighbouring blocks reuse (419 -> 434 us per call without).
+  if constexpr (CT == 1) {
+    const int32_t col = col0 + wave * 32 + (lane & 31);
+    if (col < a.N) {
 #pragma unroll
-  for (int ct = 0; ct < CT; ++ct) {
-    const int32_t col = col0 + (wave * CT + ct) * 32 + (lane & 31);
-    if (col >= a.N) continue;
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int32_t i = rt * 32 + (r & 3) + 4 * (lane >> 5) + 8 * (r >> 2);
+          if (i < rows)
+            __builtin_nontemporal_store(acc[rt][0][r], &a.C[(int64_t)(r0 + i) * a.ldc + col]);
+        }
+    }
+  } else {
+    // 256-column panels go through LDS, 16 rows at a time, so that a wave
+    // stores a row's 1 KB with 16-byte stores instead of 128-byte pieces of two
+    // rows (banded BF16, direct / so: 1M^2 N = 256 467 / 419 us per call, where
+    // copies reach this kernel's 2.0 GB in 424 us; 400000^2 N = 200 224 / 158;
+    // panels of 128 columns 291 / 295)
+    constexpr int32_t kCStride = kCols + 4;
+    float *sc = reinterpret_cast<float *>(sh.A);  // over A and B, both consumed
+    static_assert(sizeof(sh.A) + sizeof(sh.B) >= 16 * kCStride * sizeof(float),
+                  "16 rows of C fit");
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int32_t i = rt * 32 + (r & 3) + 4 * (lane >> 5) + 8 * (r >> 2);
-        if (i < rows) __builtin_nontemporal_store(acc[rt][ct][r], &a.C[(int64_t)(r0 + i) * a.ldc + col]);
+      for (int h = 0; h < 2; ++h) {
+        __syncthreads();  // the last chunk consumed / the previous rows stored
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+          for (int r = 8 * h; r < 8 * h + 8; ++r)
+            sc[((r & 3) + 4 * (lane >> 5) + 8 * ((r >> 2) & 1)) * kCStride +
+               (wave * CT + ct) * 32 + (lane & 31)] = acc[rt][ct][r];
+        __syncthreads();
+        for (int i = tid; i < 16 * kCols / 4; i += kBlockThreads) {
+          const int32_t row = rt * 32 + 16 * h + i / (kCols / 4), c = i % (kCols / 4) * 4;
+          if (row >= rows || col0 + c >= a.N) continue;
+          const f4 v = *reinterpret_cast<const f4 *>(&sc[i / (kCols / 4) * kCStride + c]);
+          float *dst = &a.C[(int64_t)(r0 + row) * a.ldc + col0 + c];
+          if (col0 + c + 4 <= a.N) {
+            __builtin_nontemporal_store(v, reinterpret_cast<f4u *>(dst));
+          } else {
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+              if (col0 + c + j < a.N) __builtin_nontemporal_store(v[j], dst + j);
+          }
+        }
       }
   }
   return true;
 }
 
-template <int DT, int CT, int RB>
+template <int DT, int CT, int RB, bool kFull8>
 __global__ __launch_bounds__(kBlockThreads) void k_bd(const KArgs a) {
   __shared__ BdShared<CT, RB> sh;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -373,7 +413,7 @@ __global__ __launch_bounds__(kBlockThreads) void k_bd(const KArgs a) {
   if constexpr (RB == 2) {
     const int32_t lo = min(sh.win[0], sh.win[2]), hi = max(sh.win[1], sh.win[3]);
     if (hi >= 0 && hi - lo + 1 <= kBdMaxW2) {
-      if (!bd_mfma<DT, CT, RB, 2>(a, sh, sh.pos, r0, rows, col0, lo, hi, kBdStride2))
+      if (!bd_mfma<DT, CT, RB, 2, kFull8>(a, sh, sh.pos, r0, rows, col0, lo, hi, kBdStride2))
         bd_rows_valu<DT>(a, r0, rows, col0, kCols);
       return;
     }
@@ -384,7 +424,7 @@ __global__ __launch_bounds__(kBlockThreads) void k_bd(const KArgs a) {
     const int32_t lo = sh.win[2 * h], hi = sh.win[2 * h + 1];
     // no entries (every row written as zeros) or too wide for the tile
     if (hi < 0 || hi - lo + 1 > kBdMaxW ||
-        !bd_mfma<DT, CT, RB, 1>(a, sh, sh.pos + 32 * h, hr0, hrows, col0, lo, hi, kBdStride1))
+        !bd_mfma<DT, CT, RB, 1, kFull8>(a, sh, sh.pos + 32 * h, hr0, hrows, col0, lo, hi, kBdStride1))
       bd_rows_valu<DT>(a, hr0, hrows, col0, kCols);
   }
 }
@@ -392,6 +432,20 @@ __global__ __launch_bounds__(kBlockThreads) void k_bd(const KArgs a) {
 }  // namespace
 
 int32_t bd_col_tiles(int32_t N) { return N > kWavesPerBlock * 32 ? 2 : 1; }
+
+template <int DT, int CT, int RB>
+static void launch_bd_t(const KArgs &a, dim3 g, dim3 b, hipStream_t s) {
+  // Odd widths read their whole 8-column segments at element alignment. The
+  // forms are two kernels because the odd one's registers would cost the
+  // other a workgroup per CU (banded 1M^2 BF16, N = 256: 420 -> 460 us per call
+  // with one kernel for both).
+  const bool full8 = (reinterpret_cast<uintptr_t>(a.B) & 15) == 0 && (a.ldb & 7) == 0 &&
+                     (a.N & 7) == 0;
+  if (full8)
+    hipLaunchKernelGGL((k_bd<DT, CT, RB, true>), g, b, 0, s, a);
+  else
+    hipLaunchKernelGGL((k_bd<DT, CT, RB, false>), g, b, 0, s, a);
+}
 
 hipError_t launch_bd(int dt, const KArgs &a, hipStream_t s) {
   const int64_t units = (int64_t)a.nblocks * a.panels;
@@ -403,14 +457,14 @@ hipError_t launch_bd(int dt, const KArgs &a, hipStream_t s) {
   const int ct = bd_col_tiles(a.N);
   const int rb = a.tile / kBdRows;
   switch (dt * 16 + ct * 4 + rb) {
-    case 1 * 16 + 1 * 4 + 1: hipLaunchKernelGGL((k_bd<1, 1, 1>), g, b, 0, s, a); break;
-    case 1 * 16 + 2 * 4 + 1: hipLaunchKernelGGL((k_bd<1, 2, 1>), g, b, 0, s, a); break;
-    case 2 * 16 + 1 * 4 + 1: hipLaunchKernelGGL((k_bd<2, 1, 1>), g, b, 0, s, a); break;
-    case 2 * 16 + 2 * 4 + 1: hipLaunchKernelGGL((k_bd<2, 2, 1>), g, b, 0, s, a); break;
-    case 1 * 16 + 1 * 4 + 2: hipLaunchKernelGGL((k_bd<1, 1, 2>), g, b, 0, s, a); break;
-    case 1 * 16 + 2 * 4 + 2: hipLaunchKernelGGL((k_bd<1, 2, 2>), g, b, 0, s, a); break;
-    case 2 * 16 + 1 * 4 + 2: hipLaunchKernelGGL((k_bd<2, 1, 2>), g, b, 0, s, a); break;
-    case 2 * 16 + 2 * 4 + 2: hipLaunchKernelGGL((k_bd<2, 2, 2>), g, b, 0, s, a); break;
+    case 1 * 16 + 1 * 4 + 1: launch_bd_t<1, 1, 1>(a, g, b, s); break;
+    case 1 * 16 + 2 * 4 + 1: launch_bd_t<1, 2, 1>(a, g, b, s); break;
+    case 2 * 16 + 1 * 4 + 1: launch_bd_t<2, 1, 1>(a, g, b, s); break;
+    case 2 * 16 + 2 * 4 + 1: launch_bd_t<2, 2, 1>(a, g, b, s); break;
+    case 1 * 16 + 1 * 4 + 2: launch_bd_t<1, 1, 2>(a, g, b, s); break;
+    case 1 * 16 + 2 * 4 + 2: launch_bd_t<1, 2, 2>(a, g, b, s); break;
+    case 2 * 16 + 1 * 4 + 2: launch_bd_t<2, 1, 2>(a, g, b, s); break;
+    case 2 * 16 + 2 * 4 + 2: launch_bd_t<2, 2, 2>(a, g, b, s); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
