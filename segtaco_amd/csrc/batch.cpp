@@ -81,7 +81,7 @@ int32_t tune_item(const segtaco_batch_item_t &it, int32_t dt,
 namespace segtaco {
 
 void fill_batch_desc(const segtaco_csr_t &A, const void *B, int64_t ldb,
-                     float *C, int64_t ldc, int32_t N,
+                     float *C, int64_t ldc, int32_t N, int32_t b_dtype,
                      const segtaco_plan_t &plan, BatchDesc *D, int64_t *units,
                      int64_t *fix_units, size_t *lds, EbLayout *lay) {
   std::memset(D, 0, sizeof(*D));
@@ -99,35 +99,36 @@ void fill_batch_desc(const segtaco_csr_t &A, const void *B, int64_t ldb,
   a.b_off32 = b_off32_ok(A.K, ldb, 4);
   a.C = C;
   a.ldc = ldc;
-  a.lq = ilog2(plan.col_lanes);
+  const ExecForm form = exec_form(plan, A.M, A.nnz, N, b_dtype, false);
+  a.lq = form.lq;
   a.lg = ilog2(plan.group);
   a.tile = plan.tile;
   a.comp_threshold = plan.comp_threshold == 0 ? INT_MAX : plan.comp_threshold;
-  a.panels = (int32_t)ceil_div(N, (int64_t)plan.col_lanes * plan.vec);
+  a.panels = form.panels;
   D->schedule = plan.schedule;
-  D->vec = plan.vec;
+  D->vec = form.vec;
   *fix_units = 0;
   *lds = 0;
   switch (plan.schedule) {
     case SEGTACO_RB_SR:
       a.nblocks = (int32_t)ceil_div(
-          A.M, (int64_t)kWavesPerBlock * (64 / plan.col_lanes) * plan.group);
+          A.M, (int64_t)kWavesPerBlock * (64 / form.lanes) * plan.group);
       break;
     case SEGTACO_RB_PR:
       a.nblocks = (int32_t)ceil_div(
-          A.M, (int64_t)(64 / (plan.col_lanes * plan.group)) * kWavesPerBlock);
+          A.M, (int64_t)(64 / (form.lanes * plan.group)) * kWavesPerBlock);
       break;
     default: {
       *lay = eb_layout(A.nnz, N, plan.tile);
       a.ntiles = lay->ntiles;
       a.rows_per_slice = (int32_t)ceil_div(A.M, lay->ntiles);
       const int64_t tiles_per_group_block =
-          (int64_t)kWavesPerBlock * (64 / plan.col_lanes);
+          (int64_t)kWavesPerBlock * (64 / form.lanes);
       a.nblocks = plan.schedule == SEGTACO_EB_SR
                       ? (int32_t)ceil_div(lay->ntiles, tiles_per_group_block)
                       : (int32_t)ceil_div(lay->ntiles, kWavesPerBlock);
       *lds = plan.schedule == SEGTACO_EB_SR ? eb_sr_lds_bytes(a)
-             : spmv_form(a, plan.vec)        ? kSvLdsBytes
+             : spmv_form(a, form.vec)        ? kSvLdsBytes
                                              : eb_pr_lds_bytes(a);
       *fix_units = ceil_div(lay->ntiles, tiles_per_group_block) * a.panels;
       break;
@@ -211,7 +212,7 @@ int32_t segtaco_batch_create(const segtaco_batch_item_t *items, int32_t n,
     b->plans[i] = plan;
     int64_t units = 0, fix_units = 0;
     size_t lds = 0;
-    fill_batch_desc(A, it.B, it.ldb, it.C, it.ldc, it.N, plan, &D, &units,
+    fill_batch_desc(A, it.B, it.ldb, it.C, it.ldc, it.N, b_dtype, plan, &D, &units,
                     &fix_units, &lds, &lay[i]);
     if (lds > b->lds) b->lds = lds;
     b->sv = b->sv || batch_uses_spmv(D);

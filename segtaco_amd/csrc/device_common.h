@@ -119,15 +119,26 @@ struct RawT<DT, 2> { using type = uint32_t; };
 template <int DT>
 struct RawT<DT, 1> { using type = uint16_t; };
 
+// A slice starts at any element: the last lane's columns end at N (lane_col)
+// and rows of odd leading dimensions start anywhere. gfx950 reads 8- and
+// 16-byte vectors from memory at any element alignment.
 template <int DT, int V>
 __device__ __forceinline__ typename RawT<DT, V>::type load_raw(
     const void *__restrict__ base, int64_t i) {
-  using R = typename RawT<DT, V>::type;
-  if constexpr (DT == 0) {
-    return *reinterpret_cast<const R *>(static_cast<const float *>(base) + i);
-  } else {
-    return *reinterpret_cast<const R *>(static_cast<const uint16_t *>(base) + i);
-  }
+  constexpr int kEb = DT == 0 ? 4 : 2;
+  typename RawT<DT, V>::type x;
+  __builtin_memcpy(&x, __builtin_assume_aligned(static_cast<const char *>(base) + i * kEb, kEb),
+                   sizeof(x));
+  return x;
+}
+
+// First column of the slice of lane `lane` of a panel row whose nominal slice
+// is [nominal, nominal + V): moved back to end at N, so that no lane reads or
+// writes past the row (V <= N). The columns it shares with its left neighbour
+// get the same value from both.
+template <int V>
+__device__ __forceinline__ int32_t lane_col(int32_t nominal, int32_t N) {
+  return min(nominal, N - V);
 }
 
 template <int DT, int V>
@@ -174,8 +185,10 @@ __device__ __forceinline__ typename RawT<DT, V>::type load_row_raw(
   if constexpr (kOff32) {
     constexpr uint32_t kEb = DT == 0 ? 4 : 2;
     const uint32_t off = (__umul24((uint32_t)row, (uint32_t)ld) + (uint32_t)c) * kEb;
-    return *reinterpret_cast<const typename RawT<DT, V>::type *>(
-        static_cast<const char *>(base) + off);
+    typename RawT<DT, V>::type x;
+    __builtin_memcpy(&x, __builtin_assume_aligned(static_cast<const char *>(base) + off, kEb),
+                     sizeof(x));
+    return x;
   } else {
     return load_raw<DT, V>(base, (int64_t)row * ld + c);
   }
@@ -221,7 +234,17 @@ __device__ __forceinline__ int32_t wave_scan(int32_t x) {
   return row == 0 ? x : op(x, row == 1 ? b1 : row == 2 ? b2 : b3);
 }
 
-// V consecutive FP32 values to C (aligned to V floats; V == 8 is two float4).
+// V consecutive FP32 values to memory, at any float alignment.
+template <int V>
+__device__ __forceinline__ void store_row(float *p, const float (&v)[V]) {
+  __builtin_memcpy(__builtin_assume_aligned(p, 4), v, sizeof(v));
+}
+template <int V>
+__device__ __forceinline__ void load_row_f32(const float *p, float (&v)[V]) {
+  __builtin_memcpy(v, __builtin_assume_aligned(p, 4), sizeof(v));
+}
+
+// V consecutive FP32 values (aligned to V floats; V == 8 is two float4).
 template <int V>
 __device__ __forceinline__ void store_vec(float *__restrict__ p,
                                           const float (&v)[V]) {
@@ -237,12 +260,12 @@ __device__ __forceinline__ void store_vec(float *__restrict__ p,
   }
 }
 
-// store_vec for data nothing reads back soon (non-temporal: not kept in L2),
+// store_row for data nothing reads back soon (non-temporal: not kept in L2),
 // as whole 16- / 8-byte vector stores.
 template <int V>
-__device__ __forceinline__ void store_vec_nt(float *__restrict__ p, const float (&v)[V]) {
-  typedef float f4 __attribute__((ext_vector_type(4)));
-  typedef float f2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void store_row_nt(float *__restrict__ p, const float (&v)[V]) {
+  typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
+  typedef float f2 __attribute__((ext_vector_type(2), aligned(4)));
   if constexpr (V == 8) {
     __builtin_nontemporal_store(f4{v[0], v[1], v[2], v[3]}, reinterpret_cast<f4 *>(p));
     __builtin_nontemporal_store(f4{v[4], v[5], v[6], v[7]}, reinterpret_cast<f4 *>(p) + 1);

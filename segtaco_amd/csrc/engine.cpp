@@ -159,6 +159,13 @@ int32_t natural_lanes(int32_t N, int32_t vec) {
   return (int32_t)(q > 64 ? 64 : q);
 }
 
+// Widest per-lane vector of N columns at any alignment (lane_col).
+int32_t widest_any(int32_t dt, int32_t N) {
+  int32_t v = dt == SEGTACO_DT_F32 ? 4 : 8;
+  while (v > 1 && v > N) v >>= 1;
+  return v;
+}
+
 int32_t resolve(const segtaco_csr_t *A, int32_t N, int32_t b_dtype,
                 int64_t ldb, int64_t ldc, const void *B, const void *C,
                 segtaco_plan_t *plan) {
@@ -307,13 +314,84 @@ int32_t check_csr(const segtaco_csr_t *A) {
 
 }  // namespace
 
+// The vector width and lanes a resolved plan runs with; no choice here changes
+// a sum's order.
+//
+// A plan's vec divides N and the leading dimensions, so an odd width would run
+// with one element per lane and load, in several panels; the kernels take a
+// row's columns in wider slices, the last one moved back to end at N
+// (lane_col). The width is the smallest that takes the row in one panel: of
+// the plan's lanes for the schedules whose lanes and slots fill the wave
+// (their slots stay), of half a wave for eb_sr, whose groups then share it,
+// and for rb_sr where a whole wave does not take the row. Measured at N = 77,
+// us per call, one element per load / so: eb_sr 50021^2 (1 M entries) FP16
+// 116 / 66, FP32 110 / 71; rb_pr of even rows FP16 104 / 38; eb_pr 153 / 97;
+// eb_cs FP32 200000^2 458 / 229. On products that leave the chip short of
+// workgroups the narrow slices' extra lanes are faster (1000^2 N = 77 eb_sr
+// 29 / 34), so those keep the plan's width.
+//
+// eb_sr alone also takes narrower slices than the plan's widest, so that a
+// group has 17 to 32 lanes: two groups per wave end their rows at different
+// steps where eight or sixteen do with the widest (power-law, tile 128, us per
+// call, widest / so: 60000^2 BF16 N = 16 138 / 46, N = 32 96 / 49, N = 128 69 /
+// 59; FP32 N = 16 80 / 47; 262144^2 BF16 N = 64 151 / 123, FP32 N = 32 129 /
+// 112; slices of one element lose from 1.2 M entries on at N > 16: 262144^2
+// N = 32 FP32 125, two elements 112). In a batch the kernel's occupancy is
+// that of its heaviest body, and wide slices keep more bytes in flight.
+ExecForm exec_form(const segtaco_plan_t &p, int32_t M, int32_t nnz, int32_t N,
+                   int32_t b_dtype, bool alone) {
+  ExecForm f{p.vec, p.col_lanes, 0, 1};
+  const int32_t w = widest_any(b_dtype, N);
+  // plans that spread a row over all the lanes it can use
+  const bool natural = p.col_lanes == natural_lanes(N, p.vec);
+  int64_t items = 0;  // lane groups of the launch
+  switch (p.schedule) {
+    case SEGTACO_RB_SR:
+      if (natural && 64 * f.vec < N) {
+        while (f.vec < w && 32 * f.vec < N) f.vec <<= 1;
+        f.lanes = natural_lanes(N, f.vec);
+      }
+      items = M;
+      break;
+    case SEGTACO_EB_SR:
+      if (natural) {
+        if (alone) f.vec = N > 16 && nnz > 1200000 ? 2 : 1;
+        while (f.vec < w && f.vec < (alone ? 4 : 8) && 32 * f.vec < N) f.vec <<= 1;
+        f.lanes = natural_lanes(N, f.vec);
+      }
+      items = ceil_div(nnz, p.tile);
+      break;
+    case SEGTACO_RB_PR:
+      while (f.vec < w && f.lanes * f.vec < N) f.vec <<= 1;
+      items = (int64_t)M * p.group;
+      break;
+    case SEGTACO_EB_PR:
+      while (f.vec < w && f.lanes * f.vec < N) f.vec <<= 1;
+      items = ceil_div(nnz, p.tile) * p.group;
+      break;
+    case SEGTACO_EB_CS:  // LDS slots of lanes * vec floats, vec at most 4
+      while (f.vec < w && f.vec < 4 && f.lanes * f.vec < N) f.vec <<= 1;
+      items = INT64_MAX / 64;
+      break;
+    default:
+      break;
+  }
+  if (f.vec > p.vec && items * f.lanes < 2 * (int64_t)device_cus() * kBlockThreads) {
+    f.vec = p.vec;
+    f.lanes = p.col_lanes;
+  }
+  f.lq = ilog2(f.lanes);
+  f.panels = (int32_t)ceil_div(N, (int64_t)f.lanes * f.vec);
+  return f;
+}
+
 namespace {
 
 // Workspace of a plan whose tile, group and vec are all set.
 size_t resolved_workspace_bytes(const segtaco_csr_t *A, int32_t N,
                                 const segtaco_plan_t &p, int32_t b_dtype) {
   if (p.schedule == SEGTACO_EB_CS)
-    return cs_layout(A->nnz, A->K, N, p.tile, p.group, p.vec).total;
+    return cs_layout(A->nnz, A->K, N, p.tile, p.group, exec_form(p, A->M, A->nnz, N, b_dtype, true).vec).total;
   if (p.schedule != SEGTACO_EB_SR && p.schedule != SEGTACO_EB_PR) return 0;
   return eb_layout(A->nnz, N, p.tile).total;
 }
@@ -377,7 +455,8 @@ int32_t cs_workspace_layout_impl(const segtaco_csr_t *A, int32_t N,
                      "segtaco_cs_workspace_layout: schedule %d is not eb_cs", plan->schedule);
   if (plan->tile < 8 || plan->vec < 1 || plan->group < 1)
     return set_error(SEGTACO_ERR_INVALID, "segtaco_cs_workspace_layout: unresolved plan");
-  const CsLayout L = cs_layout(A->nnz, A->K, N, plan->tile, plan->group, plan->vec);
+  const CsLayout L = cs_layout(A->nnz, A->K, N, plan->tile, plan->group,
+                               exec_form(*plan, A->M, A->nnz, N, SEGTACO_DT_F32, true).vec);
   const int64_t v[10] = {L.units, L.cap, L.packed,
                          (int64_t)L.rec_off, (int64_t)L.rows_off, (int64_t)L.int_off,
                          (int64_t)L.code_off, (int64_t)L.nslot_off, (int64_t)L.count_off,
@@ -493,12 +572,16 @@ int32_t spmm_impl(const segtaco_csr_t *A, const void *B, int32_t b_dtype,
   a.b_off32 = b_off32_ok(A->K, ldb, elem_bytes(b_dtype));
   a.C = C;
   a.ldc = ldc;
-  a.lq = ilog2(plan.col_lanes);
-  a.lg = ilog2(plan.group);
+  const ExecForm form = exec_form(plan, A->M, A->nnz, N, b_dtype, true);
+  const int32_t V = form.vec;
+  a.lq = form.lq;
+  // rb_sr's rows per group only order the launch: one row per group keeps
+  // more rows in flight (uniform 100003 x 90001, 20 entries per row, N = 32
+  // FP32: 42 -> 36 us against two rows, BF16 30 -> 22)
+  a.lg = plan.schedule == SEGTACO_RB_SR ? 0 : ilog2(plan.group);
   a.tile = plan.tile;
   a.comp_threshold = plan.comp_threshold == 0 ? INT_MAX : plan.comp_threshold;
-  const int32_t V = plan.vec;
-  a.panels = (int32_t)ceil_div(N, (int64_t)plan.col_lanes * V);
+  a.panels = form.panels;
 
   auto mark = [&](int i) -> hipError_t {
     return ev ? hipEventRecord(ev[i], stream) : hipSuccess;
@@ -506,8 +589,7 @@ int32_t spmm_impl(const segtaco_csr_t *A, const void *B, int32_t b_dtype,
   switch (plan.schedule) {
     case SEGTACO_RB_SR: {
       if (!run) return SEGTACO_OK;  // nothing depends on A alone
-      const int64_t rows_per_block =
-          (int64_t)kWavesPerBlock * (64 / plan.col_lanes) * plan.group;
+      const int64_t rows_per_block = (int64_t)kWavesPerBlock * (64 / form.lanes);
       a.nblocks = (int32_t)ceil_div(A->M, rows_per_block);
       SEGTACO_HIP(mark(0));
       SEGTACO_HIP(mark(1));
@@ -518,7 +600,7 @@ int32_t spmm_impl(const segtaco_csr_t *A, const void *B, int32_t b_dtype,
     }
     case SEGTACO_RB_PR: {
       if (!run) return SEGTACO_OK;  // nothing depends on A alone
-      const int64_t rows_per_wave = 64 / (plan.col_lanes * plan.group);
+      const int64_t rows_per_wave = 64 / (form.lanes * plan.group);
       a.nblocks = (int32_t)ceil_div(A->M, rows_per_wave * kWavesPerBlock);
       SEGTACO_HIP(mark(0));
       SEGTACO_HIP(mark(1));
@@ -625,7 +707,7 @@ int32_t spmm_impl(const segtaco_csr_t *A, const void *B, int32_t b_dtype,
   a.tile_row = reinterpret_cast<int32_t *>(w + L.rows_off);
   if (prepare) prep_record(ws, nullptr);
   SEGTACO_HIP(mark(0));
-  const int64_t tiles_per_block = (int64_t)kWavesPerBlock * (64 / plan.col_lanes);
+  const int64_t tiles_per_block = (int64_t)kWavesPerBlock * (64 / form.lanes);
   if (run && plan.schedule == SEGTACO_EB_SR) {
     SegArgs g;
     if (const int32_t sv =

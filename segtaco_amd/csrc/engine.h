@@ -87,6 +87,14 @@ int32_t plan_resolve_ptrs_impl(const segtaco_csr_t *A, int32_t N, int32_t b_dtyp
                                int64_t ldb, int64_t ldc, const void *B, const void *C,
                                segtaco_plan_t *plan);
 
+// The vector width and lanes per B row a resolved plan runs with, in a call
+// of its own (alone) or in a batch.
+struct ExecForm {
+  int32_t vec, lanes, lq, panels;
+};
+ExecForm exec_form(const segtaco_plan_t &p, int32_t M, int32_t nnz, int32_t N,
+                   int32_t b_dtype, bool alone);
+
 // Default element-balanced tile of a product with nnz entries: `tile`,
 // halved (not below 8) while the product would have fewer than two
 // workgroups of `tiles_per_block` tiles per compute unit. Each lane group

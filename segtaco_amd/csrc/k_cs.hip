@@ -465,7 +465,7 @@ struct CsBatch {
 
 // The pipelined loop shared by the sweep and the walk over entries [s, e):
 // Every load is unconditional (entries past the tile re-read its last
-// entry; columns past N read column 0; neither is used), so the loads in
+// entry; lanes past N its last columns; neither is used), so the loads in
 // flight are the same on every path and each wait covers only its batch:
 // loads complete in issue order, and per iteration the metadata of batch
 // b + 2 goes out before the gathers of batch b + 1, so waiting for the
@@ -524,11 +524,10 @@ __device__ __forceinline__ void cs_sweep(const CsArgs &a, float *acc_lds, int32_
   struct G {
     R b[kB];
   };
-  const int32_t col_ld = colok ? col : 0;
   auto gather = [&](const M &m, G &g) {
 #pragma unroll
     for (int u = 0; u < kB; ++u)
-      g.b[u] = load_raw<DT, V>(a.B, (int64_t)m.c[u] * a.ldb + col_ld);
+      g.b[u] = load_raw<DT, V>(a.B, (int64_t)m.c[u] * a.ldb + col);
   };
   auto consume = [&](const M &m, const G &g, int32_t i0) {
     const int32_t nb = min(kB, e - i0);
@@ -564,12 +563,11 @@ __device__ __forceinline__ void cs_walk(const CsArgs &a, int32_t t, int32_t s, i
     R b[kB];
     int32_t row[kB];
   };
-  const int32_t col_ld = colok ? col : 0;
   const int32_t *rows = a.int_rows + (int64_t)t * a.tile;
   auto gather = [&](const M &m, G &g) {
 #pragma unroll
     for (int u = 0; u < kB; ++u) {
-      g.b[u] = load_raw<DT, V>(a.B, (int64_t)m.c[u] * a.ldb + col_ld);
+      g.b[u] = load_raw<DT, V>(a.B, (int64_t)m.c[u] * a.ldb + col);
       g.row[u] = rows[max(m.s[u] - 2, 0)];
     }
   };
@@ -581,7 +579,7 @@ __device__ __forceinline__ void cs_walk(const CsArgs &a, int32_t t, int32_t s, i
     float *dst = cur == 0   ? a.carry_head + (int64_t)t * a.N + col
                  : cur == 1 ? a.carry_tail + (int64_t)t * a.N + col
                             : a.C + (int64_t)row * a.ldc + col;
-    store_vec<V>(dst, acc);
+    store_row<V>(dst, acc);
   };
   auto consume = [&](const M &m, const G &g, int32_t i0) {
     const int32_t nb = min(kB, e - i0);
@@ -659,8 +657,9 @@ __global__ __launch_bounds__(kCsThreads) void k_eb_cs(const CsArgs a) {
     float z[V];
     zero_vec(z);
     for (int32_t panel = 0; panel < panels; ++panel) {
-      const int32_t col = panel * W + q * V;
-      const bool colok = col < a.N;
+      const int32_t nominal = panel * W + q * V;
+      const bool colok = nominal < a.N;
+      const int32_t col = lane_col<V>(nominal, a.N);
       if (walk)
         cs_walk<DT, V, kPacked>(a, t, s, e, col, colok);
       else
@@ -674,13 +673,13 @@ __global__ __launch_bounds__(kCsThreads) void k_eb_cs(const CsArgs a) {
         if (head_carry) {
 #pragma unroll
           for (int k = 0; k < V; ++k) x[k] = acc_lds[(2 * g) * W + q * V + k];
-          store_vec<V>(a.carry_head + (int64_t)t * a.N + col, x);
+          store_row<V>(a.carry_head + (int64_t)t * a.N + col, x);
           store_vec<V>(acc_lds + (2 * g) * W + q * V, z);
         }
         if (tail_carry) {
 #pragma unroll
           for (int k = 0; k < V; ++k) x[k] = acc_lds[(2 * g + 1) * W + q * V + k];
-          store_vec<V>(a.carry_tail + (int64_t)t * a.N + col, x);
+          store_row<V>(a.carry_tail + (int64_t)t * a.N + col, x);
           store_vec<V>(acc_lds + (2 * g + 1) * W + q * V, z);
         }
         if (fold_t0 >= 0) {
@@ -695,7 +694,7 @@ __global__ __launch_bounds__(kCsThreads) void k_eb_cs(const CsArgs a) {
             for (int k = 0; k < V; ++k) x[k] += sl[k];
             store_vec<V>(sl, z);
           }
-          store_vec<V>(a.C + (int64_t)fold_row * a.ldc + col, x);
+          store_row<V>(a.C + (int64_t)fold_row * a.ldc + col, x);
         }
       }
       // interior slots to C
@@ -710,7 +709,7 @@ __global__ __launch_bounds__(kCsThreads) void k_eb_cs(const CsArgs a) {
           float x[V];
 #pragma unroll
           for (int k = 0; k < V; ++k) x[k] = acc_lds[sl * W + seg * V + k];
-          store_vec<V>(a.C + (int64_t)row * a.ldc + c, x);
+          store_row<V>(a.C + (int64_t)row * a.ldc + lane_col<V>(c, a.N), x);
           store_vec<V>(acc_lds + sl * W + seg * V, z);
         }
       }

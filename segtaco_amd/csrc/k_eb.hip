@@ -88,7 +88,7 @@ __global__ __launch_bounds__(kBlockThreads) void k_tile_rows_fix(
     const int i = __ffsll(m) - 1;
     m &= m - 1;
     float *row = C + (wave_row0 + i) * ldc;
-    for (int32_t j = lane * V; j < N; j += 64 * V) store_vec<V>(row + j, z);
+    for (int32_t j = lane * V; j < N; j += 64 * V) store_row<V>(row + lane_col<V>(j, N), z);
   }
 }
 

@@ -16,9 +16,9 @@
 //   * all lanes gather the range's B slices, entry after entry, whatever row
 //     they belong to, into LDS (column-major, FP32);
 //   * the range's pieces (row x tile) are listed in LDS, and lane groups of
-//     one lane per column (two above 64 columns) sum them from there, each
-//     taking the next piece as it finishes its last. A piece's sum is a
-//     serial chain of up to T steps, but of LDS reads instead of gathers.
+//     one lane per column sum them from there, each taking the next piece as
+//     it finishes its last. A piece's sum is a serial chain of up to T steps,
+//     but of LDS reads instead of gathers.
 // The sums and folds are those of eb_sr for the same T, bit for bit: a
 // piece is summed sequentially, the pieces of a row that begins and ends in
 // the range are folded in order; a row that began before the range stores
@@ -45,7 +45,6 @@
 namespace segtaco {
 namespace {
 
-constexpr int kSegU = kSegStep;
 constexpr int kSegG = 16;  // gathers per lane in flight before they go to LDS
 
 // Flags of a segment or piece beside its start (ranges are at most 1024 long).
@@ -53,32 +52,6 @@ constexpr uint32_t kSegStart = 0x3ff;
 constexpr uint32_t kSegComp = 0x8000;   // of a compensated row
 constexpr uint32_t kSegMany = 0x4000;   // of a segment over several tiles
 constexpr uint32_t kSegFirst = 0x2000;  // the segment's first piece
-
-// A B slice at any element alignment: the last lane's columns are moved back
-// to end at N, so a slice need not start at a multiple of V elements, and
-// rows of odd leading dimensions start at any element. gfx950 reads 8- and
-// 16-byte vectors at element alignment.
-template <int DT, int V, bool kOff32>
-__device__ __forceinline__ typename RawT<DT, V>::type seg_load(const void *__restrict__ base,
-                                                               int32_t row, int64_t ld,
-                                                               int32_t c) {
-  constexpr uint32_t kEb = DT == 0 ? 4 : 2;
-  const char *p;
-  if constexpr (kOff32)
-    p = static_cast<const char *>(base) +
-        (__umul24((uint32_t)row, (uint32_t)ld) + (uint32_t)c) * kEb;
-  else
-    p = static_cast<const char *>(base) + ((int64_t)row * ld + c) * kEb;
-  typename RawT<DT, V>::type x;
-  __builtin_memcpy(&x, __builtin_assume_aligned(p, kEb), sizeof(x));
-  return x;
-}
-
-// V floats at any float alignment.
-template <int V>
-__device__ __forceinline__ void seg_store(float *p, const float (&v)[V]) {
-  __builtin_memcpy(__builtin_assume_aligned(p, 4), v, sizeof(v));
-}
 
 // Last row r in [lo, hi) with pos[r] <= target, given pos[lo] <= target <
 // pos[hi]: 64 probes per step. The whole wave calls it; the result is uniform.
@@ -119,8 +92,7 @@ __device__ __forceinline__ void wave_rows_of(const int32_t *__restrict__ pos, in
   r1 = l1;
 }
 
-// Sums: W columns per lane (1, or 2 for more than 64 columns).
-template <int DT, int V, int W, bool kOff32, bool kComp>
+template <int DT, int V, bool kOff32, bool kComp>
 __global__ __launch_bounds__(64) void k_eb_seg(const SegArgs g) {
   extern __shared__ __align__(16) char smem[];
   using R = typename RawT<DT, V>::type;
@@ -133,7 +105,7 @@ __global__ __launch_bounds__(64) void k_eb_seg(const SegArgs g) {
   const int32_t q = lane & (Q - 1);
   const int32_t grp = lane >> lq;
   const bool colok = q * V < a.N;
-  const int32_t col = min(q * V, a.N - V);  // V <= N
+  const int32_t col = lane_col<V>(q * V, a.N);
   const int32_t P = seg_pad(g.range), sx = seg_stride(g.range);
   float *s_x = reinterpret_cast<float *>(smem);  // [Q * V][sx]: column-major
   float *s_val = s_x + ((size_t)(V * sx) << lq);
@@ -144,8 +116,8 @@ __global__ __launch_bounds__(64) void k_eb_seg(const SegArgs g) {
   uint16_t *s_pk = s_pc + P;
   // several tiles per range: sums of the pieces of segments over several
   // tiles, [first piece, tile], then [later piece, tile]; and those segments
-  float *s_sum = reinterpret_cast<float *>(s_seg + 4 * P);  // [2 * tpr][W << ls]
-  uint16_t *s_many = reinterpret_cast<uint16_t *>(s_sum + ((size_t)(2 * g.tpr * W) << g.ls));
+  float *s_sum = reinterpret_cast<float *>(s_seg + 4 * P);  // [2 * tpr][1 << ls]
+  uint16_t *s_many = reinterpret_cast<uint16_t *>(s_sum + ((size_t)(2 * g.tpr) << g.ls));
 
   const int32_t *__restrict__ pos = a.pos;
   const int32_t T = a.tile;
@@ -166,7 +138,7 @@ __global__ __launch_bounds__(64) void k_eb_seg(const SegArgs g) {
   };
   auto gather = [&]() {
 #pragma unroll
-    for (int u = 0; u < kSegG; ++u) x[u] = seg_load<DT, V, kOff32>(a.B, c[u], a.ldb, col);
+    for (int u = 0; u < kSegG; ++u) x[u] = load_row_raw<DT, V, kOff32>(a.B, c[u], a.ldb, col);
   };
   auto stage = [&](int32_t i0) {
 #pragma unroll
@@ -207,7 +179,7 @@ __global__ __launch_bounds__(64) void k_eb_seg(const SegArgs g) {
       if (m == 0) continue;
       for (int32_t i = 0; i < Q; ++i) {
         const int32_t b = i * G + grp;
-        if (((m >> b) & 1) && colok) seg_store<V>(a.C + (r + b) * a.ldc + col, z);
+        if (((m >> b) & 1) && colok) store_row<V>(a.C + (r + b) * a.ldc + col, z);
       }
     }
   }
@@ -296,26 +268,19 @@ __global__ __launch_bounds__(64) void k_eb_seg(const SegArgs g) {
     wave_sync();
   }
 
-  // 5. sums: lane groups of one lane per W columns take the pieces in order,
-  // each the next one as it finishes its last; a step reads an aligned block
-  // of eight entries (two 16-byte reads per column and two of the values).
+  // 5. sums: lane groups of one lane per column take the pieces in order, each
+  // the next one as it finishes its last; a step reads an aligned block of
+  // eight entries (two 16-byte reads of the column and two of the values).
   const int ls = g.ls;
   const int32_t L = 1 << ls;
   const int32_t l = lane & (L - 1);
   const int32_t sg = lane >> ls;
-  const bool ok = l * W < a.N;
-  const int32_t scol = min(l * W, a.N - W);
-  // where the gather put columns scol .. scol + W - 1 (its last lane's slice
-  // ends at N)
-  const float *xc[W];
-#pragma unroll
-  for (int j = 0; j < W; ++j) {
-    const int32_t whole = a.N / V * V, cj = scol + j;
-    xc[j] = s_x + (cj < whole ? cj : cj - a.N + V + whole) * sx;
-  }
-  float acc[W], cmp[W];
-  zero_vec(acc);
-  zero_vec(cmp);
+  const bool ok = l < a.N;
+  const int32_t scol = min(l, a.N - 1);
+  // where the gather put column scol (its last lane's slice ends at N)
+  const int32_t whole = a.N / V * V;
+  const float *xc = s_x + (scol < whole ? scol : scol - a.N + V + whole) * sx;
+  float acc = 0.0f, cmp = 0.0f;
   const uint64_t leaders = __ballot(l == 0);
   const uint64_t below = ((uint64_t)1 << (lane & ~(L - 1))) - 1;
   int32_t nxt = 0;
@@ -334,53 +299,40 @@ __global__ __launch_bounds__(64) void k_eb_seg(const SegArgs g) {
           gf = s_pc[p];
           gi = (int32_t)(gf & kSegStart);
           ge = p + 1 < np ? (int32_t)(s_pc[p + 1] & kSegStart) : cn;
-          zero_vec(acc);
-          zero_vec(cmp);
+          acc = cmp = 0.0f;
         }
       }
       if (!__ballot(gi < ge)) break;
     }
     if (gi < ge) {
-      const int32_t i0 = gi & ~(kSegU - 1);
-      const uint32_t lo = (uint32_t)(gi - i0), n = (uint32_t)min(ge - i0, kSegU) - lo;
-      float v[kSegU], xv[W][kSegU];
-      load_f32vec<kSegU>(s_val + i0, v);
-#pragma unroll
-      for (int j = 0; j < W; ++j) load_f32vec<kSegU>(xc[j] + i0, xv[j]);
+      const int32_t i0 = gi & ~(kSegStep - 1);
+      const uint32_t lo = (uint32_t)(gi - i0), n = (uint32_t)min(ge - i0, kSegStep) - lo;
+      float v[kSegStep], x[kSegStep];
+      load_f32vec<kSegStep>(s_val + i0, v);
+      load_f32vec<kSegStep>(xc + i0, x);
       if (kComp && (gf & kSegComp)) {
 #pragma unroll
-        for (int u = 0; u < kSegU; ++u) {
-          if (u - lo < n) {
-#pragma unroll
-            for (int j = 0; j < W; ++j) neumaier_add(acc[j], cmp[j], v[u], xv[j][u]);
-          }
-        }
+        for (int u = 0; u < kSegStep; ++u)
+          if (u - lo < n) neumaier_add(acc, cmp, v[u], x[u]);
       } else {
 #pragma unroll
-        for (int u = 0; u < kSegU; ++u) {
-#pragma unroll
-          for (int j = 0; j < W; ++j) {
-            const float t = fmaf(v[u], xv[j][u], acc[j]);
-            acc[j] = u - lo < n ? t : acc[j];
-          }
+        for (int u = 0; u < kSegStep; ++u) {
+          const float t = fmaf(v[u], x[u], acc);
+          acc = u - lo < n ? t : acc;
         }
       }
-      gi = i0 + kSegU;
+      gi = i0 + kSegStep;
       if (gi >= ge) {
-        if (kComp && (gf & kSegComp)) {
-#pragma unroll
-          for (int j = 0; j < W; ++j) acc[j] += cmp[j];
-        }
+        if (kComp && (gf & kSegComp)) acc += cmp;
         const int32_t k = g.tpr > 1 ? (int32_t)s_pk[gp] : gp;
         if (head && k == 0) {
-          if (ok) seg_store<W>(a.carry_head + (int64_t)((s0 + ge - 1) / T) * a.N + scol, acc);
+          if (ok) a.carry_head[(int64_t)((s0 + ge - 1) / T) * a.N + scol] = acc;
         } else if (g.tpr > 1 && (gf & kSegMany)) {
           const int32_t b = (ge - 1) / T + (gf & kSegFirst ? 0 : g.tpr);
-          store_vec<W>(s_sum + ((b << ls) + l) * W, acc);
+          s_sum[(b << ls) + l] = acc;
         } else if (ok) {
-          seg_store<W>(cross && k == nseg - 1 ? a.carry_tail + (int64_t)w * g.tpr * a.N + scol
-                                              : a.C + (int64_t)s_row[k] * a.ldc + scol,
-                       acc);
+          *(cross && k == nseg - 1 ? a.carry_tail + (int64_t)w * g.tpr * a.N + scol
+                                   : a.C + (int64_t)s_row[k] * a.ldc + scol) = acc;
         }
       }
     }
@@ -396,17 +348,11 @@ __global__ __launch_bounds__(64) void k_eb_seg(const SegArgs g) {
     const int32_t en = k + 1 < nseg ? (int32_t)(s_seg[k + 1] & kSegStart) : cn;
     const int32_t b1 = (en - 1) / T;
     int32_t b = st / T;
-    float y[W];
-    load_f32vec<W>(s_sum + ((b << ls) + l) * W, acc);
-    while (++b <= b1) {
-      load_f32vec<W>(s_sum + (((g.tpr + b) << ls) + l) * W, y);
-#pragma unroll
-      for (int j = 0; j < W; ++j) acc[j] += y[j];
-    }
+    acc = s_sum[(b << ls) + l];
+    while (++b <= b1) acc += s_sum[((g.tpr + b) << ls) + l];
     if (ok)
-      seg_store<W>(cross && k == nseg - 1 ? a.carry_tail + (int64_t)w * g.tpr * a.N + scol
-                                          : a.C + (int64_t)s_row[k] * a.ldc + scol,
-                   acc);
+      *(cross && k == nseg - 1 ? a.carry_tail + (int64_t)w * g.tpr * a.N + scol
+                               : a.C + (int64_t)s_row[k] * a.ldc + scol) = acc;
   }
 }
 
@@ -444,22 +390,22 @@ __global__ __launch_bounds__(kBlockThreads) void k_seg_fixup(const SegArgs g) {
   }
 }
 
-template <int DT, int V, int W>
+template <int DT, int V>
 hipError_t launch_seg_v(const SegArgs &g, hipStream_t s) {
   if (g.nranges <= 0) return hipSuccess;
-  const size_t lds = seg_lds_wave(g.range, g.a.lq, V, g.tpr, g.ls, W);
+  const size_t lds = seg_lds_wave(g.range, g.a.lq, V, g.tpr, g.ls);
   const dim3 gr((unsigned)g.nranges), b(64);
   const bool comp = g.a.comp_threshold < g.a.nnz;  // some row may be compensated
   if (g.a.b_off32) {
     if (comp)
-      hipLaunchKernelGGL((k_eb_seg<DT, V, W, true, true>), gr, b, lds, s, g);
+      hipLaunchKernelGGL((k_eb_seg<DT, V, true, true>), gr, b, lds, s, g);
     else
-      hipLaunchKernelGGL((k_eb_seg<DT, V, W, true, false>), gr, b, lds, s, g);
+      hipLaunchKernelGGL((k_eb_seg<DT, V, true, false>), gr, b, lds, s, g);
   } else {
     if (comp)
-      hipLaunchKernelGGL((k_eb_seg<DT, V, W, false, true>), gr, b, lds, s, g);
+      hipLaunchKernelGGL((k_eb_seg<DT, V, false, true>), gr, b, lds, s, g);
     else
-      hipLaunchKernelGGL((k_eb_seg<DT, V, W, false, false>), gr, b, lds, s, g);
+      hipLaunchKernelGGL((k_eb_seg<DT, V, false, false>), gr, b, lds, s, g);
   }
   return hipGetLastError();
 }
@@ -468,14 +414,12 @@ hipError_t launch_seg_v(const SegArgs &g, hipStream_t s) {
 
 template <int DT>
 hipError_t launch_seg_t(int vec, const SegArgs &g, hipStream_t s) {
-  constexpr int kWide = DT == 0 ? 4 : 8;
-  if (g.a.N > 64) return launch_seg_v<DT, kWide, 2>(g, s);
   switch (vec) {
-    case 1: return launch_seg_v<DT, 1, 1>(g, s);
-    case 2: return launch_seg_v<DT, 2, 1>(g, s);
-    case 4: return launch_seg_v<DT, 4, 1>(g, s);
+    case 1: return launch_seg_v<DT, 1>(g, s);
+    case 2: return launch_seg_v<DT, 2>(g, s);
+    case 4: return launch_seg_v<DT, 4>(g, s);
     case 8:
-      if constexpr (DT != 0) return launch_seg_v<DT, 8, 1>(g, s);
+      if constexpr (DT != 0) return launch_seg_v<DT, 8>(g, s);
       return hipErrorInvalidValue;
     default: return hipErrorInvalidValue;
   }
@@ -511,13 +455,13 @@ int32_t seg_plan(int32_t dt, const KArgs &a, int64_t walk_blocks, SegArgs *g) {
   //     144 / 95 and 129 / 95);
   //   9 to 16: 60000^2 (1 M entries) 81 / 36 and 56 / 43; 200000^2 (2.4 M) 93 /
   //     79 and 74 / 82; 262144^2 (4.2 M) 116 / 126: up to 24 M products;
-  //   17 to 128: small products (1000^2, 15.6 K entries, N = 64: 36 / 22 at
+  //   17 to 64: small products (1000^2, 15.6 K entries, N = 64: 36 / 22 at
   //     tile 128, 21 / 13 at tile 8), and where the walk leaves half of the
   //     chip without a workgroup: 8000^2 N = 64 (63 workgroups) 43 / 28, but
   //     20000^2 N = 50 (156 workgroups) 40 / 46, 60000^2 N = 64 53 / 131.
   // A range has to fit the wave's LDS, and the zero fill walks M / ranges
   // rows per wave, so mostly empty matrices keep the row-parallel partition.
-  if (a.tile > kSegMaxRange || a.N > 128 || (int64_t)a.M > 2 * (int64_t)a.nnz) return 0;
+  if (a.tile > kSegMaxRange || a.N > 64 || (int64_t)a.M > 2 * (int64_t)a.nnz) return 0;
   const int64_t products = (int64_t)a.nnz * a.N;
   const bool take = a.N <= 8    ? true
                     : a.N <= 16 ? products <= 24000000
@@ -530,17 +474,16 @@ int32_t seg_plan(int32_t dt, const KArgs &a, int64_t walk_blocks, SegArgs *g) {
   while (v > a.N) v >>= 1;
   s.a.lq = 0;
   while ((v << s.a.lq) < a.N) ++s.a.lq;
-  const int W = a.N > 64 ? 2 : 1;
   s.ls = 0;
-  while ((W << s.ls) < a.N) ++s.ls;
+  while ((1 << s.ls) < a.N) ++s.ls;
   // about 2048 entries per lane of a group, but at least 2048 waves
-  int64_t want = std::min(std::max(2048 / (W << s.ls), 128), 384);
+  int64_t want = std::min(std::max(2048 >> s.ls, 128), 384);
   want = std::min(want, ceil_div64(a.nnz, 2048));
   s.tpr = (int32_t)std::max<int64_t>(1, want / a.tile);
   s.range = s.tpr * a.tile;
   s.nranges = (int32_t)ceil_div64(a.nnz, s.range);
   s.slice = (int32_t)ceil_div64(a.M, s.nranges);
-  if (seg_lds_wave(s.range, s.a.lq, v, s.tpr, s.ls, W) > 65536) return 0;
+  if (seg_lds_wave(s.range, s.a.lq, v, s.tpr, s.ls) > 65536) return 0;
   return v;
 }
 #endif

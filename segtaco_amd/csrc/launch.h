@@ -21,12 +21,12 @@ struct KArgs {
   int64_t ldb;
   float *C;
   int64_t ldc;
-  int32_t lq;              // log2(col_lanes): lanes per B-row segment
+  int32_t lq;              // log2 of the lanes per B-row segment (exec_form)
   int32_t lg;              // log2(group): *_pr nnz slots per row / pass
   int32_t tile;            // eb_*: nnz per tile
   int32_t ntiles;          // eb_*: ceil(nnz / tile)
   int32_t comp_threshold;  // rows longer than this are compensated
-  int32_t panels;          // column panels: ceil(N / (col_lanes * vec))
+  int32_t panels;          // column panels: ceil(N / (lanes * vec))
   int32_t nblocks;         // row / tile blocks before panel expansion
   int32_t rows_per_slice;  // eb_*: rows per tile for empty-row zero fill
   const int32_t *part;     // eb_*: K21 partition, ntiles + 1 entries
@@ -117,7 +117,7 @@ hipError_t launch_batch_fixup(const BatchDesc *d, int32_t n,
 // element-balanced pointers (part, tile_row, carries) are left null.
 struct EbLayout;
 void fill_batch_desc(const segtaco_csr_t &A, const void *B, int64_t ldb,
-                     float *C, int64_t ldc, int32_t N,
+                     float *C, int64_t ldc, int32_t N, int32_t b_dtype,
                      const segtaco_plan_t &plan, BatchDesc *D, int64_t *units,
                      int64_t *fix_units, size_t *lds, EbLayout *lay);
 // Workgroups of the persistent launch that fit the device at once.

@@ -89,7 +89,7 @@ __device__ __forceinline__ void zero_empty_rows(const KArgs &a, int32_t r0,
       float *crow = a.C + (int64_t)r * a.ldc;
       for (int32_t qq = 0; qq < Q; ++qq) {
         const int32_t cc = ((panel << a.lq) + qq) * V;
-        if (cc < a.N) store_vec<V>(crow + cc, z);
+        if (cc < a.N) store_row<V>(crow + lane_col<V>(cc, a.N), z);
       }
     }
   }
@@ -123,8 +123,9 @@ __device__ __forceinline__ void eb_sr_walk(const KArgs &a, int32_t blk,
   const void *__restrict__ vals = a.vals;
   const void *__restrict__ B = a.B;
   const int64_t ldb = a.ldb;
-  const int32_t col = ((panel << lq) + q) * V;
-  const bool colok = col < a.N;
+  const int32_t nominal = ((panel << lq) + q) * V;
+  const bool colok = nominal < a.N;
+  const int32_t col = lane_col<V>(nominal, a.N);
   const bool tok = t < a.ntiles;
   const int32_t s = tok ? t * a.tile : 0;
   const int32_t e =
@@ -154,10 +155,10 @@ __device__ __forceinline__ void eb_sr_walk(const KArgs &a, int32_t blk,
     }
     if (before || after) {
       // carries: read back by the fix-up
-      store_vec<V>((before ? a.carry_head : a.carry_tail) + (int64_t)t * a.N + col, acc);
+      store_row<V>((before ? a.carry_head : a.carry_tail) + (int64_t)t * a.N + col, acc);
     } else {
       // C rows are never read back here: non-temporal, to leave L2 to B
-      store_vec_nt<V>(a.C + (int64_t)r * a.ldc + col, acc);
+      store_row_nt<V>(a.C + (int64_t)r * a.ldc + col, acc);
     }
   };
   auto next_row = [&](int32_t pp) {
@@ -198,17 +199,16 @@ __device__ __forceinline__ void eb_sr_walk(const KArgs &a, int32_t blk,
       // Double-buffered: batch k+1's gathers are in flight while batch k is
       // consumed, so the memory pipe never drains between batches. Every
       // batch issues exactly kSrBatch loads, with no branch around them
-      // (entries past the chunk and columns past N re-load the chunk's last
-      // entry / column 0, and are not consumed): the number of loads in flight
+      // (entries past the chunk re-load its last one and lanes past N its last
+      // columns, and are not consumed): the number of loads in flight
       // is then the same on every path, so the wait before consuming a batch
       // only covers that batch and leaves the next one in flight.
       R ra[kSrBatch], rb[kSrBatch];
-      const int32_t col_ld = colok ? col : 0;
       auto issue = [&](R (&buf)[kSrBatch], int32_t b0) {
 #pragma unroll
         for (int u = 0; u < kSrBatch; ++u) {
           const int32_t i = min(b0 + u, cn - 1);
-          buf[u] = load_row_raw<DT, V, kOff32>(B, s_crd[i], ldb, col_ld);
+          buf[u] = load_row_raw<DT, V, kOff32>(B, s_crd[i], ldb, col);
         }
       };
       auto consume = [&](const R (&buf)[kSrBatch], int32_t b0) {
@@ -327,8 +327,9 @@ __device__ __forceinline__ void eb_pr_walk(const KArgs &a, int32_t blk,
   const void *__restrict__ vals = a.vals;
   const void *__restrict__ B = a.B;
   const int64_t ldb = a.ldb;
-  const int32_t col = ((panel << lq) + q) * V;
-  const bool colok = col < a.N;
+  const int32_t nominal = ((panel << lq) + q) * V;
+  const bool colok = nominal < a.N;
+  const int32_t col = lane_col<V>(nominal, a.N);
   const int32_t s = t * a.tile;
   const int32_t e = (int32_t)min((int64_t)a.nnz, (int64_t)s + a.tile);
   // Upper bound on the rows of this tile: the row holding entry e (M when
@@ -367,14 +368,13 @@ __device__ __forceinline__ void eb_pr_walk(const KArgs &a, int32_t blk,
 #pragma unroll
       for (int u = 0; u < kPrPasses; ++u) {
         // every pass issues its load, with no branch around it (slots past
-        // the chunk re-load its last entry, columns past N column 0), so the
-        // wait before a pass covers only that pass's load
+        // the chunk re-load its last entry, lanes past N its last columns), so
+        // the wait before a pass covers only that pass's load
         const int32_t i = pb + u * P + sl;
         const bool ok = i < cn;
         rid[u] = ok ? s_row[i] : INT_MAX;
         vv[u] = ok ? s_val[i] : 0.0f;
-        raw[u] = load_row_raw<DT, V, kOff32>(B, s_crd[min(i, cn - 1)], ldb,
-                                             colok ? col : 0);
+        raw[u] = load_row_raw<DT, V, kOff32>(B, s_crd[min(i, cn - 1)], ldb, col);
       }
 #pragma unroll
       for (int u = 0; u < kPrPasses; ++u) {
@@ -417,7 +417,7 @@ __device__ __forceinline__ void eb_pr_walk(const KArgs &a, int32_t blk,
           float *dst = before  ? a.carry_head + (int64_t)t * a.N + col
                        : after ? a.carry_tail + (int64_t)t * a.N + col
                                : a.C + (int64_t)my * a.ldc + col;
-          store_vec<V>(dst, prod);
+          store_row<V>(dst, prod);
         }
         if (last_open) {
 #pragma unroll
@@ -463,14 +463,14 @@ __device__ __forceinline__ void combine_carries(const KArgs &a, int32_t t0,
                                                 int32_t t, int32_t r,
                                                 int32_t col) {
   float acc[V];
-  load_f32vec<V>(a.carry_tail + (int64_t)t0 * a.N + col, acc);
+  load_row_f32<V>(a.carry_tail + (int64_t)t0 * a.N + col, acc);
   constexpr int kH = 8;
   int32_t tt = t0 + 1;
   for (; tt + kH - 1 <= t; tt += kH) {
     float h[kH][V];
 #pragma unroll
     for (int k = 0; k < kH; ++k)
-      load_f32vec<V>(a.carry_head + (int64_t)(tt + k) * a.N + col, h[k]);
+      load_row_f32<V>(a.carry_head + (int64_t)(tt + k) * a.N + col, h[k]);
 #pragma unroll
     for (int k = 0; k < kH; ++k)
 #pragma unroll
@@ -478,11 +478,11 @@ __device__ __forceinline__ void combine_carries(const KArgs &a, int32_t t0,
   }
   for (; tt <= t; ++tt) {
     float h[V];
-    load_f32vec<V>(a.carry_head + (int64_t)tt * a.N + col, h);
+    load_row_f32<V>(a.carry_head + (int64_t)tt * a.N + col, h);
 #pragma unroll
     for (int j = 0; j < V; ++j) acc[j] += h[j];
   }
-  store_vec<V>(a.C + (int64_t)r * a.ldc + col, acc);
+  store_row<V>(a.C + (int64_t)r * a.ldc + col, acc);
 }
 
 // Per tile t (one lane group). With a.fix_t0 (standalone calls, where
@@ -500,10 +500,11 @@ __device__ __forceinline__ void fixup_body(const KArgs &a, int32_t blk,
   const int32_t q = lane & (Q - 1);
   const int32_t t = ((blk * kWavesPerBlock + wave) << (6 - lq)) + (lane >> lq);
   if (t >= a.ntiles) return;
-  const int32_t col = ((panel << lq) + q) * V;
+  const int32_t nominal = ((panel << lq) + q) * V;
+  const int32_t col = lane_col<V>(nominal, a.N);
   if (a.fix_t0) {
     const int32_t t0 = a.fix_t0[t];
-    if (t0 < 0 || col >= a.N) return;
+    if (t0 < 0 || nominal >= a.N) return;
     // eb_cs has already written the rows it could sum from its LDS slots
     if (a.cs_flags && cs_row_folded(a.cs_flags, a.cs_group, t0, t)) return;
     combine_carries<V>(a, t0, t, a.tile_row[t], col);
@@ -514,7 +515,7 @@ __device__ __forceinline__ void fixup_body(const KArgs &a, int32_t blk,
     const int64_t r1 = r0 + a.rows_per_slice < a.M ? r0 + a.rows_per_slice : a.M;
     if (r0 < r1) zero_empty_rows<V>(a, (int32_t)r0, (int32_t)r1, q, Q, panel);
   }
-  if (t == 0 || col >= a.N) return;
+  if (t == 0 || nominal >= a.N) return;
   const int32_t *__restrict__ pos = a.pos;
   const int32_t s = t * a.tile;
   const int32_t e = (int32_t)min((int64_t)a.nnz, (int64_t)s + a.tile);

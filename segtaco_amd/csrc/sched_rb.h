@@ -73,7 +73,7 @@ __device__ __forceinline__ void rb_sr_row(const KArgs &a, int32_t row,
       for (int j = 0; j < V; ++j) acc[j] = fmaf(v, b[j], acc[j]);
     }
   }
-  store_vec<V>(a.C + (int64_t)row * a.ldc + col, acc);
+  store_row<V>(a.C + (int64_t)row * a.ldc + col, acc);
 }
 
 // rb_sr over row block `blk`, column panel `panel`: lane group gi owns rows
@@ -86,8 +86,9 @@ __device__ __forceinline__ void rb_sr_walk(const KArgs &a, int32_t blk,
   const int lq = a.lq;
   const int32_t gi =
       ((blk * kWavesPerBlock + wave) << (6 - lq)) + (lane >> lq);
-  const int32_t col = ((panel << lq) + (lane & ((1 << lq) - 1))) * V;
-  if (col >= a.N) return;
+  const int32_t nominal = ((panel << lq) + (lane & ((1 << lq) - 1))) * V;
+  if (nominal >= a.N) return;
+  const int32_t col = lane_col<V>(nominal, a.N);
   const int64_t first = (int64_t)gi << a.lg;
   const int32_t R = 1 << a.lg;
   for (int32_t i = 0; i < R; ++i) {
@@ -119,8 +120,9 @@ __device__ __forceinline__ void rb_pr_walk(const KArgs &a, int32_t blk,
   const int32_t row = row0 + (lane >> (lq + lg));
   const int32_t slot = (lane >> lq) & ((1 << lg) - 1);
   const int32_t P = 1 << lg;
-  const int32_t col = ((panel << lq) + (lane & ((1 << lq) - 1))) * V;
-  const bool live = row < a.M && col < a.N;
+  const int32_t nominal = ((panel << lq) + (lane & ((1 << lq) - 1))) * V;
+  const int32_t col = lane_col<V>(nominal, a.N);
+  const bool live = row < a.M && nominal < a.N;
 
   float acc[V];
   zero_vec(acc);
@@ -176,7 +178,7 @@ __device__ __forceinline__ void rb_pr_walk(const KArgs &a, int32_t blk,
 #pragma unroll
     for (int j = 0; j < V; ++j) acc[j] += __shfl_xor(acc[j], d << lq, 64);
   }
-  if (live && slot == 0) store_vec<V>(a.C + (int64_t)row * a.ldc + col, acc);
+  if (live && slot == 0) store_row<V>(a.C + (int64_t)row * a.ldc + col, acc);
 }
 
 template <int DT, int V>

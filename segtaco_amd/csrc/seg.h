@@ -33,11 +33,11 @@ __host__ __device__ inline int32_t seg_stride(int32_t range) {
 
 // LDS of one wave: the gathered B slices (vec << lq columns, FP32), per entry
 // the value and 12 bytes of segment and piece lists; with several tiles per
-// range two sums (w << ls floats) per tile and a list entry.
+// range two sums (1 << ls floats) per tile and a list entry.
 __host__ __device__ inline size_t seg_lds_wave(int32_t range, int32_t lq, int vec, int32_t tpr,
-                                               int32_t ls, int w) {
+                                               int32_t ls) {
   const size_t b = ((size_t)vec << lq) * seg_stride(range) * 4 + (size_t)seg_pad(range) * 16 +
-                   (tpr > 1 ? (size_t)tpr * (8 * ((size_t)w << ls) + 4) : 0);
+                   (tpr > 1 ? (size_t)tpr * (8 * ((size_t)1 << ls) + 4) : 0);
   return (b + 15) & ~(size_t)15;
 }
 

@@ -446,7 +446,8 @@ void launch_tick(segtaco_server *s, int32_t si) {
     int64_t units = 0, fix = 0;
     size_t l = 0;
     EbLayout lay{};
-    fill_batch_desc(A, r.B, r.ldb, r.C, r.ldc, r.N, r.plan, &D, &units, &fix, &l, &lay);
+    fill_batch_desc(A, r.B, r.ldb, r.C, r.ldc, r.N, s->cfg.dtype, r.plan, &D, &units, &fix,
+                    &l, &lay);
     if (r.plan.schedule >= SEGTACO_EB_SR && m.nnz > 0) {
       D.a.part = trs[i].part;
       D.a.tile_row = trs[i].rows;

@@ -42,7 +42,7 @@ def _structure(name, rng):
 
 @pytest.mark.parametrize("N,dtype", [(1, "f32"), (2, "bf16"), (3, "f32"), (4, "f32"), (5, "fp16"),
                                      (8, "bf16"), (16, "f32"), (17, "f32"), (33, "bf16"),
-                                     (64, "f32"), (65, "f32"), (73, "fp16"), (128, "bf16")])
+                                     (63, "fp16"), (64, "f32")])
 @pytest.mark.parametrize("tile", [8, 33, 128, 384, 1024])
 def test_same_bits_as_the_walk(N, dtype, tile):
     t = torch()
