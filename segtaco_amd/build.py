@@ -33,17 +33,17 @@ COMMON = [
 ]
 
 # (source, object name, extra flags): the batched and element-balanced
-# kernels are compiled once per storage type (and, for the batch, per N = 1
-# form), so those objects build in parallel instead of in one long pass.
+# kernels are compiled once per storage type (and, for the batch, per
+# set of schedules), so those objects build in parallel instead of in one long pass.
 LIB_SOURCES = (
     [(s, os.path.splitext(s)[0], []) for s in (
         "k_rb.hip", "k_eb.hip", "k_batch.hip", "engine.cpp", "legacy.cpp", "legacy_cxx.cpp",
         "gen.cpp", "autotune.cpp", "batch.cpp", "serve.cpp", "io.cpp", "vendor.cpp",
         "k_sddmm.hip", "sddmm.cpp", "k_cs.hip", "k_spmv.hip", "k_bd.hip", "staging.cpp",
         "noalloc.hip")]
-    + [("k_batch_inst.hip", f"k_batch_{dt}_{sv}",
-        [f"-DSEGTACO_BATCH_DT={dt}", f"-DSEGTACO_BATCH_SV={sv}"])
-       for dt in range(3) for sv in range(2)]
+    + [("k_batch_inst.hip", f"k_batch_{dt}_{form}",
+        [f"-DSEGTACO_BATCH_DT={dt}", f"-DSEGTACO_BATCH_FORM={form}"])
+       for dt in range(3) for form in range(3)]
     + [("k_eb_inst.hip", f"k_eb_{dt}", [f"-DSEGTACO_EB_DT={dt}"]) for dt in range(3)]
     + [("k_seg.hip", f"k_seg_{dt}", [f"-DSEGTACO_SEG_DT={dt}"]) for dt in range(3)]
 )

@@ -7,6 +7,7 @@
 // persistent launch over all units, one batched fix-up launch. The sequence
 // can be captured into a HIP graph (no memset nodes: the counter is cleared
 // by a kernel).
+#include <algorithm>
 #include <climits>
 #include <cstring>
 #include <vector>
@@ -37,7 +38,7 @@ struct segtaco_batch {
   size_t ws_bytes = 0;
   size_t lds = 0;
   int32_t grid = 0;
-  bool sv = false;  // some product runs the N = 1 form of eb_pr
+  BatchForm form = kBatchEbSr;  // the largest of its products'
   hipStream_t cap_stream = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -99,7 +100,7 @@ void fill_batch_desc(const segtaco_csr_t &A, const void *B, int64_t ldb,
   a.b_off32 = b_off32_ok(A.K, ldb, 4);
   a.C = C;
   a.ldc = ldc;
-  const ExecForm form = exec_form(plan, A.M, A.nnz, N, b_dtype, false);
+  const ExecForm form = exec_form(plan, A.M, A.nnz, N, b_dtype);
   a.lq = form.lq;
   a.lg = ilog2(plan.group);
   a.tile = plan.tile;
@@ -215,7 +216,7 @@ int32_t segtaco_batch_create(const segtaco_batch_item_t *items, int32_t n,
     fill_batch_desc(A, it.B, it.ldb, it.C, it.ldc, it.N, b_dtype, plan, &D, &units,
                     &fix_units, &lds, &lay[i]);
     if (lds > b->lds) b->lds = lds;
-    b->sv = b->sv || batch_uses_spmv(D);
+    b->form = std::max(b->form, batch_form(D));
     if (plan.schedule >= SEGTACO_EB_SR) {
       ws_off[i] = ws_total;
       ws_total += align_up(lay[i].total, 256);
@@ -272,7 +273,7 @@ int32_t segtaco_batch_create(const segtaco_batch_item_t *items, int32_t n,
   if ((e = hipMemcpy(b->d_fix_prefix, b->fix_prefix.data(), sizeof(int64_t) * (n + 1),
                      hipMemcpyHostToDevice)) != hipSuccess)
     return fail(e, "hipMemcpy(fix prefix)");
-  if ((e = batch_main_grid(b_dtype, b->lds, &b->grid, b->sv)) != hipSuccess)
+  if ((e = batch_main_grid(b_dtype, b->lds, &b->grid, b->form)) != hipSuccess)
     return fail(e, "batch_main_grid");
   if ((e = hipStreamSynchronize(stream)) != hipSuccess) return fail(e, "hipStreamSynchronize");
   *out = b;
@@ -285,7 +286,7 @@ int32_t segtaco_batch_run(segtaco_batch_t b, void *stream_v) {
   if (b->n == 0) return SEGTACO_OK;
   SEGTACO_HIP(launch_batch_main(b->dt, b->d_desc, b->n, b->d_prefix, b->total_units,
                                 b->d_counter, b->grid, b->lds, s, /*reset_counter=*/true,
-                                b->sv));
+                                b->form));
   SEGTACO_HIP(launch_batch_fixup(b->d_desc, b->n, b->d_fix_prefix, b->total_fix, s));
   return SEGTACO_OK;
 }

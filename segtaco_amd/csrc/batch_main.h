@@ -1,6 +1,6 @@
 // batch_main.h — the persistent batched kernel over a list of heterogeneous
-// SpMMs, as a template over the storage type (DT) and whether the N = 1 form
-// of eb_pr is compiled in (kSv). Each (DT, kSv) pair is instantiated in its
+// SpMMs, as a template over the storage type (DT) and the schedules that are
+// compiled in (kForm, BatchForm). Each (DT, kForm) pair is instantiated in its
 // own translation unit (k_batch_inst.hip, compiled once per pair) so the
 // pairs compile in parallel; k_batch.hip dispatches between them.
 //
@@ -34,11 +34,11 @@ __device__ __forceinline__ int32_t find_product(const int64_t *prefix,
   return lo;
 }
 
-// Occupancy-sized grid and launch of k_batch_main<DT, kSv> (defined in
+// Occupancy-sized grid and launch of k_batch_main<DT, kForm> (defined in
 // k_batch_inst.hip, one instantiation per object file).
-template <int DT, bool kSv>
+template <int DT, BatchForm kForm>
 hipError_t batch_main_grid_t(size_t lds, int32_t *grid);
-template <int DT, bool kSv>
+template <int DT, BatchForm kForm>
 hipError_t launch_batch_main_t(const BatchDesc *d, int32_t n,
                                const int64_t *prefix, int64_t total,
                                unsigned long long *counter, int32_t grid,

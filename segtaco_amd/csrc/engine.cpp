@@ -330,16 +330,17 @@ int32_t check_csr(const segtaco_csr_t *A) {
 // workgroups the narrow slices' extra lanes are faster (1000^2 N = 77 eb_sr
 // 29 / 34), so those keep the plan's width.
 //
-// eb_sr alone also takes narrower slices than the plan's widest, so that a
+// eb_sr also takes narrower slices than the plan's widest, so that a
 // group has 17 to 32 lanes: two groups per wave end their rows at different
 // steps where eight or sixteen do with the widest (power-law, tile 128, us per
 // call, widest / so: 60000^2 BF16 N = 16 138 / 46, N = 32 96 / 49, N = 128 69 /
 // 59; FP32 N = 16 80 / 47; 262144^2 BF16 N = 64 151 / 123, FP32 N = 32 129 /
 // 112; slices of one element lose from 1.2 M entries on at N > 16: 262144^2
-// N = 32 FP32 125, two elements 112). In a batch the kernel's occupancy is
-// that of its heaviest body, and wide slices keep more bytes in flight.
+// N = 32 FP32 125, two elements 112). So do its products in a batch (12 power-law
+// products of 2000 to 20000 rows: BF16 N <= 64 286 / 119, FP32 N <= 64 164 / 118;
+// 24 of up to 200000 rows, FP32 N <= 128 2440 / 2320).
 ExecForm exec_form(const segtaco_plan_t &p, int32_t M, int32_t nnz, int32_t N,
-                   int32_t b_dtype, bool alone) {
+                   int32_t b_dtype) {
   ExecForm f{p.vec, p.col_lanes, 0, 1};
   const int32_t w = widest_any(b_dtype, N);
   // plans that spread a row over all the lanes it can use
@@ -355,8 +356,8 @@ ExecForm exec_form(const segtaco_plan_t &p, int32_t M, int32_t nnz, int32_t N,
       break;
     case SEGTACO_EB_SR:
       if (natural) {
-        if (alone) f.vec = N > 16 && nnz > 1200000 ? 2 : 1;
-        while (f.vec < w && f.vec < (alone ? 4 : 8) && 32 * f.vec < N) f.vec <<= 1;
+        f.vec = N > 16 && nnz > 1200000 ? 2 : 1;
+        while (f.vec < w && f.vec < 4 && 32 * f.vec < N) f.vec <<= 1;
         f.lanes = natural_lanes(N, f.vec);
       }
       items = ceil_div(nnz, p.tile);
@@ -391,7 +392,9 @@ namespace {
 size_t resolved_workspace_bytes(const segtaco_csr_t *A, int32_t N,
                                 const segtaco_plan_t &p, int32_t b_dtype) {
   if (p.schedule == SEGTACO_EB_CS)
-    return cs_layout(A->nnz, A->K, N, p.tile, p.group, exec_form(p, A->M, A->nnz, N, b_dtype, true).vec).total;
+    return cs_layout(A->nnz, A->K, N, p.tile, p.group,
+                     exec_form(p, A->M, A->nnz, N, b_dtype).vec)
+        .total;
   if (p.schedule != SEGTACO_EB_SR && p.schedule != SEGTACO_EB_PR) return 0;
   return eb_layout(A->nnz, N, p.tile).total;
 }
@@ -456,7 +459,7 @@ int32_t cs_workspace_layout_impl(const segtaco_csr_t *A, int32_t N,
   if (plan->tile < 8 || plan->vec < 1 || plan->group < 1)
     return set_error(SEGTACO_ERR_INVALID, "segtaco_cs_workspace_layout: unresolved plan");
   const CsLayout L = cs_layout(A->nnz, A->K, N, plan->tile, plan->group,
-                               exec_form(*plan, A->M, A->nnz, N, SEGTACO_DT_F32, true).vec);
+                               exec_form(*plan, A->M, A->nnz, N, SEGTACO_DT_F32).vec);
   const int64_t v[10] = {L.units, L.cap, L.packed,
                          (int64_t)L.rec_off, (int64_t)L.rows_off, (int64_t)L.int_off,
                          (int64_t)L.code_off, (int64_t)L.nslot_off, (int64_t)L.count_off,
@@ -572,7 +575,7 @@ int32_t spmm_impl(const segtaco_csr_t *A, const void *B, int32_t b_dtype,
   a.b_off32 = b_off32_ok(A->K, ldb, elem_bytes(b_dtype));
   a.C = C;
   a.ldc = ldc;
-  const ExecForm form = exec_form(plan, A->M, A->nnz, N, b_dtype, true);
+  const ExecForm form = exec_form(plan, A->M, A->nnz, N, b_dtype);
   const int32_t V = form.vec;
   a.lq = form.lq;
   // rb_sr's rows per group only order the launch: one row per group keeps

@@ -93,7 +93,7 @@ struct ExecForm {
   int32_t vec, lanes, lq, panels;
 };
 ExecForm exec_form(const segtaco_plan_t &p, int32_t M, int32_t nnz, int32_t N,
-                   int32_t b_dtype, bool alone);
+                   int32_t b_dtype);
 
 // Default element-balanced tile of a product with nnz entries: `tile`,
 // halved (not below 8) while the product would have fewer than two

@@ -27,34 +27,38 @@ __global__ __launch_bounds__(kBlockThreads) void k_batch_fixup(
   }
 }
 
-hipError_t batch_main_grid(int dt, size_t lds, int32_t *grid, bool sv) {
-  switch (dt * 2 + (sv ? 1 : 0)) {
-    case 0: return batch_main_grid_t<0, false>(lds, grid);
-    case 1: return batch_main_grid_t<0, true>(lds, grid);
-    case 2: return batch_main_grid_t<1, false>(lds, grid);
-    case 3: return batch_main_grid_t<1, true>(lds, grid);
-    case 4: return batch_main_grid_t<2, false>(lds, grid);
-    case 5: return batch_main_grid_t<2, true>(lds, grid);
-    default: return hipErrorInvalidValue;
+// RUN(DT, kForm) for the pair (dt, form)
+#define SEGTACO_BATCH_FORMS(DT, RUN)       \
+  switch (form) {                          \
+    case kBatchEbSr: RUN(DT, kBatchEbSr);  \
+    case kBatchAny: RUN(DT, kBatchAny);    \
+    case kBatchSv: RUN(DT, kBatchSv);      \
+    default: return hipErrorInvalidValue;  \
   }
+#define SEGTACO_BATCH_DISPATCH(RUN)        \
+  switch (dt) {                            \
+    case 0: SEGTACO_BATCH_FORMS(0, RUN)    \
+    case 1: SEGTACO_BATCH_FORMS(1, RUN)    \
+    case 2: SEGTACO_BATCH_FORMS(2, RUN)    \
+    default: return hipErrorInvalidValue;  \
+  }
+
+hipError_t batch_main_grid(int dt, size_t lds, int32_t *grid, BatchForm form) {
+#define RUN(DT, F) return batch_main_grid_t<DT, F>(lds, grid)
+  SEGTACO_BATCH_DISPATCH(RUN)
+#undef RUN
 }
 
 hipError_t launch_batch_main(int dt, const BatchDesc *d, int32_t n,
                              const int64_t *prefix, int64_t total,
                              unsigned long long *counter, int32_t grid,
-                             size_t lds, hipStream_t s, bool reset_counter, bool sv) {
+                             size_t lds, hipStream_t s, bool reset_counter, BatchForm form) {
   if (reset_counter) hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(1), 0, s, counter);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || total <= 0) return e;
-  switch (dt * 2 + (sv ? 1 : 0)) {
-    case 0: return launch_batch_main_t<0, false>(d, n, prefix, total, counter, grid, lds, s);
-    case 1: return launch_batch_main_t<0, true>(d, n, prefix, total, counter, grid, lds, s);
-    case 2: return launch_batch_main_t<1, false>(d, n, prefix, total, counter, grid, lds, s);
-    case 3: return launch_batch_main_t<1, true>(d, n, prefix, total, counter, grid, lds, s);
-    case 4: return launch_batch_main_t<2, false>(d, n, prefix, total, counter, grid, lds, s);
-    case 5: return launch_batch_main_t<2, true>(d, n, prefix, total, counter, grid, lds, s);
-    default: return hipErrorInvalidValue;
-  }
+#define RUN(DT, F) return launch_batch_main_t<DT, F>(d, n, prefix, total, counter, grid, lds, s)
+  SEGTACO_BATCH_DISPATCH(RUN)
+#undef RUN
 }
 
 hipError_t launch_batch_fixup(const BatchDesc *d, int32_t n,

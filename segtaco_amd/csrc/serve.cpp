@@ -194,7 +194,7 @@ struct segtaco_server {
   std::thread th;
   bool stop = false;
   int64_t next_id = 0, use_clock = 0;
-  std::map<std::pair<size_t, bool>, int32_t> grid_by_lds;  // (LDS, N = 1 form)
+  std::map<std::pair<size_t, BatchForm>, int32_t> grid_by_lds;
   // statistics
   std::vector<double> lat_us;
   int64_t submitted = 0, completed = 0, rejected = 0, ticks = 0;
@@ -435,7 +435,7 @@ void launch_tick(segtaco_server *s, int32_t si) {
   }
   if (chosen.empty() && !issued) return;
   size_t lds = 0;
-  bool sv = false;  // some product runs the N = 1 form of eb_pr
+  BatchForm form = kBatchEbSr;  // the largest of the products'
   int64_t total = 0, total_fix = 0;
   slot.h_prefix[0] = slot.h_fix[0] = 0;
   for (size_t i = 0; i < chosen.size(); ++i) {
@@ -463,16 +463,16 @@ void launch_tick(segtaco_server *s, int32_t si) {
     slot.h_prefix[i + 1] = total;
     slot.h_fix[i + 1] = total_fix;
     lds = std::max(lds, l);
-    sv = sv || batch_uses_spmv(D);
+    form = std::max(form, batch_form(D));
     r.flops = 2.0 * m.nnz * r.N;
   }
   const int32_t n = (int32_t)chosen.size();
   int32_t grid = 1;
-  auto g = s->grid_by_lds.find({lds, sv});
+  auto g = s->grid_by_lds.find({lds, form});
   if (g != s->grid_by_lds.end()) {
     grid = g->second;
-  } else if (batch_main_grid(s->cfg.dtype, lds, &grid, sv) == hipSuccess) {
-    s->grid_by_lds[{lds, sv}] = grid;
+  } else if (batch_main_grid(s->cfg.dtype, lds, &grid, form) == hipSuccess) {
+    s->grid_by_lds[{lds, form}] = grid;
   } else {
     grid = 1024;
   }
@@ -486,7 +486,8 @@ void launch_tick(segtaco_server *s, int32_t si) {
                        hipMemcpyHostToDevice, slot.stream);
   if (e == hipSuccess && n > 0)
     e = launch_batch_main(s->cfg.dtype, slot.d_desc, n, slot.d_prefix, total,
-                          slot.d_counter, grid, lds, slot.stream, /*reset_counter=*/false, sv);
+                          slot.d_counter, grid, lds, slot.stream, /*reset_counter=*/false,
+                          form);
   if (e == hipSuccess && n > 0)
     e = launch_batch_fixup(slot.d_desc, n, slot.d_fix, total_fix, slot.stream);
   if (e == hipSuccess) e = hipEventRecord(slot.done, slot.stream);

@@ -26,9 +26,10 @@ __host__ __device__ inline bool spmv_form(const KArgs &a, int vec) {
          (E & (E - 1)) == 0;
 }
 inline bool spmv_applies(const KArgs &a, int vec) { return spmv_form(a, vec); }
-// Whether a batched product runs the N = 1 form.
-inline bool batch_uses_spmv(const BatchDesc &D) {
-  return D.schedule == SEGTACO_EB_PR && spmv_form(D.a, D.vec);
+// The kernel that a batched product needs.
+inline BatchForm batch_form(const BatchDesc &D) {
+  if (D.schedule == SEGTACO_EB_SR && D.vec <= 4) return kBatchEbSr;
+  return D.schedule == SEGTACO_EB_PR && spmv_form(D.a, D.vec) ? kBatchSv : kBatchAny;
 }
 
 hipError_t launch_spmv(int dt, const KArgs &a, hipStream_t s);
