@@ -113,7 +113,7 @@ void fill_batch_desc(const segtaco_csr_t &A, const void *B, int64_t ldb,
   switch (plan.schedule) {
     case SEGTACO_RB_SR:
       a.nblocks = (int32_t)ceil_div(
-          A.M, (int64_t)kWavesPerBlock * (64 / form.lanes) * plan.group);
+          A.M, (int64_t)kWavesPerBlock * (64 / form.lanes));
       break;
     case SEGTACO_RB_PR:
       a.nblocks = (int32_t)ceil_div(

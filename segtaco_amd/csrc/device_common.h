@@ -234,6 +234,52 @@ __device__ __forceinline__ int32_t wave_scan(int32_t x) {
   return row == 0 ? x : op(x, row == 1 ? b1 : row == 2 ? b2 : b3);
 }
 
+// x + (x of lane ^ D) for a power of two D < 64: row shifts and quad permutes
+// below 16 (DPP) and gfx950's half-row swaps above, no LDS shuffle
+// (ds_bpermute: an LDS access and a wait per value). Both lanes of a pair get
+// the same bits.
+template <int D>
+__device__ __forceinline__ float add_xor_lane(float x) {
+  const int32_t i = __float_as_int(x);
+  if constexpr (D >= 16) {
+    // swap(x, x): {even rows / lower half twice, odd rows / upper half twice}
+    const auto p = D == 32
+                       ? __builtin_amdgcn_permlane32_swap((uint32_t)i, (uint32_t)i, false, false)
+                       : __builtin_amdgcn_permlane16_swap((uint32_t)i, (uint32_t)i, false, false);
+    return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+  } else {
+    int32_t o;
+    if constexpr (D == 8) {
+      o = __builtin_amdgcn_update_dpp(i, i, 0x128, 0xF, 0xF, false);  // row_ror:8
+    } else if constexpr (D == 4) {
+      o = __builtin_amdgcn_update_dpp(i, i, 0x104, 0xF, 0x5, false);  // row_shl:4, banks 0, 2
+      o = __builtin_amdgcn_update_dpp(o, i, 0x114, 0xF, 0xA, false);  // row_shr:4, banks 1, 3
+    } else if constexpr (D == 2) {
+      o = __builtin_amdgcn_update_dpp(i, i, 0x4E, 0xF, 0xF, false);  // quad_perm 2,3,0,1
+    } else {
+      o = __builtin_amdgcn_update_dpp(i, i, 0xB1, 0xF, 0xF, false);  // quad_perm 1,0,3,2
+    }
+    return x + __int_as_float(o);
+  }
+}
+
+// Butterfly sums of n values over lane distances `from`, from/2, .. `to`
+// (uniform powers of two): one uniform branch per distance.
+template <int n>
+__device__ __forceinline__ void butterfly(float (&x)[n], int32_t from, int32_t to) {
+#define SEGTACO_BUTTERFLY(D_)                                    \
+  if (from >= D_ && to <= D_) {                                  \
+    _Pragma("unroll") for (int j = 0; j < n; ++j) x[j] = add_xor_lane<D_>(x[j]); \
+  }
+  SEGTACO_BUTTERFLY(32)
+  SEGTACO_BUTTERFLY(16)
+  SEGTACO_BUTTERFLY(8)
+  SEGTACO_BUTTERFLY(4)
+  SEGTACO_BUTTERFLY(2)
+  SEGTACO_BUTTERFLY(1)
+#undef SEGTACO_BUTTERFLY
+}
+
 // V consecutive FP32 values to memory, at any float alignment.
 template <int V>
 __device__ __forceinline__ void store_row(float *p, const float (&v)[V]) {

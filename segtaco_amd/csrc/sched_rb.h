@@ -6,13 +6,18 @@
 // stored entries in CSR order, gathering V-wide slices of B rows (one
 // coalesced Q*V-element request per entry) and accumulating sequentially, so
 // every C element is a sequential sum in entry order (Eigen's order, with
-// FMA). Eight entries are in flight per lane group to cover HBM/MALL latency.
+// FMA).
 //
 // rb_pr (reference: spmm_rb_pr.h:223-375, K2): P = group slots of Q lanes
 // share one row; slot s takes entries s, s+P, s+2P, ... and the P partial
 // sums are combined with a butterfly over lane distances Q..Q*P/2, a fixed
 // tree order, so results are deterministic. The reference's 32-lane,
 // 4-column warps become 64-lane waves with Q*P*R = 64.
+//
+// Both walk in batches whose gathers are in flight together. A batch's
+// columns and values are loaded during the batch before it, so a batch costs
+// one memory latency, not two; every load is unconditional, so a row's last,
+// partial batch costs one latency too, and no wait covers more than its batch.
 //
 // Neither schedule needs C cleared first: every row (empty ones included) is
 // written exactly once.
@@ -22,172 +27,283 @@
 
 namespace segtaco {
 
-// One output row of rb_sr for this lane's V columns.
-template <int DT, int V, bool kOff32>
-__device__ __forceinline__ void rb_sr_row(const KArgs &a, int32_t row,
-                                          int32_t col) {
-  const int32_t *__restrict__ crd = a.crd;
-  const void *__restrict__ vals = a.vals;
-  const void *__restrict__ B = a.B;
-  const int64_t ldb = a.ldb;
-  int32_t p = a.pos[row];
-  const int32_t e = a.pos[row + 1];
-  float acc[V];
-  zero_vec(acc);
+// acc += v * x for this lane's V columns; compensated with kComp.
+template <int DT, int V, bool kComp>
+__device__ __forceinline__ void rb_add(const typename RawT<DT, V>::type &x, float v,
+                                       float (&acc)[V], float (&cmp)[V]) {
+  float f[V];
+  unpack<DT, V>(x, f);
+#pragma unroll
+  for (int j = 0; j < V; ++j) {
+    if constexpr (kComp)
+      neumaier_add(acc[j], cmp[j], v, f[j]);
+    else
+      acc[j] = fmaf(v, f[j], acc[j]);
+  }
+}
+// The same where `on`, without a branch.
+template <int DT, int V, bool kComp>
+__device__ __forceinline__ void rb_add_if(bool on, const typename RawT<DT, V>::type &x, float v,
+                                          float (&acc)[V], float (&cmp)[V]) {
+  float s[V], t[V];
+#pragma unroll
+  for (int j = 0; j < V; ++j) {
+    s[j] = acc[j];
+    t[j] = cmp[j];
+  }
+  rb_add<DT, V, kComp>(x, v, s, t);
+#pragma unroll
+  for (int j = 0; j < V; ++j) {
+    acc[j] = on ? s[j] : acc[j];
+    if constexpr (kComp) cmp[j] = on ? t[j] : cmp[j];
+  }
+}
 
-  if (e - p > a.comp_threshold) {
-    float cmp[V];
-    zero_vec(cmp);
-    for (; p < e; ++p) {
-      float b[V];
-      const float v = load_val<DT>(vals, p);
-      load_row_vec<DT, V, kOff32>(B, crd[p], ldb, col, b);
+
+// Columns and values of a batch of U consecutive entries, as 16-byte loads
+// at element alignment (kRun: entries i .. i + U - 1 exist), or one load
+// per entry at min(i + u, last). Without values the value loads read crd (in
+// bounds: at most 4 bytes per entry) and are replaced by 1.0.
+template <int DT, bool kRun, int U>
+struct RbEntries {
+  int32_t c[U];
+  typename RawT<DT, 1>::type v[U];
+  __device__ __forceinline__ void load(const KArgs &a, int32_t i, int32_t last) {
+    constexpr int kEb = sizeof(v[0]);
+    const char *vsrc = static_cast<const char *>(a.vals ? a.vals : a.crd);
+    if constexpr (kRun) {
+      __builtin_memcpy(c, __builtin_assume_aligned(a.crd + i, 4), sizeof(c));
+      __builtin_memcpy(v, __builtin_assume_aligned(vsrc + (int64_t)i * kEb, kEb), sizeof(v));
+    } else {
 #pragma unroll
-      for (int j = 0; j < V; ++j) neumaier_add(acc[j], cmp[j], v, b[j]);
-    }
-#pragma unroll
-    for (int j = 0; j < V; ++j) acc[j] += cmp[j];
-  } else {
-    constexpr int U = (V >= 8) ? 4 : 8;
-    for (; p + U <= e; p += U) {
-      int32_t c[U];
-      float v[U];
-      float b[U][V];
-#pragma unroll
-      for (int u = 0; u < U; ++u) c[u] = crd[p + u];
-#pragma unroll
-      for (int u = 0; u < U; ++u) v[u] = load_val<DT>(vals, p + u);
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        load_row_vec<DT, V, kOff32>(B, c[u], ldb, col, b[u]);
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-#pragma unroll
-        for (int j = 0; j < V; ++j) acc[j] = fmaf(v[u], b[u][j], acc[j]);
-    }
-    for (; p < e; ++p) {
-      float b[V];
-      const float v = load_val<DT>(vals, p);
-      load_row_vec<DT, V, kOff32>(B, crd[p], ldb, col, b);
-#pragma unroll
-      for (int j = 0; j < V; ++j) acc[j] = fmaf(v, b[j], acc[j]);
+      for (int u = 0; u < U; ++u) {
+        const int32_t j = i + min(u, last - i);
+        c[u] = a.crd[j];
+        __builtin_memcpy(&v[u], __builtin_assume_aligned(vsrc + (int64_t)j * kEb, kEb), kEb);
+      }
     }
   }
+  __device__ __forceinline__ float val(const KArgs &a, int u) const {
+    if (!a.vals) return 1.0f;
+    if constexpr (DT == 0)
+      return v[u];
+    else
+      return half_to_f32<DT>(v[u]);
+  }
+};
+
+// The sum of entries p .. e - 1 (p < e) for this lane's V columns. Whole
+// batches run without a predicate on their entries; the last, partial one
+// gathers its first entry's row in the place of missing ones.
+// kRun: entries up to e + 2 * U - 2 exist.
+template <int DT, int V, bool kOff32, int U, bool kRun, bool kComp>
+__device__ __forceinline__ void rb_sr_sum(const KArgs &a, int32_t p, int32_t e, int32_t col,
+                                          float (&acc)[V]) {
+  using R = typename RawT<DT, V>::type;
+  float cmp[V];
+  zero_vec(cmp);
+  RbEntries<DT, kRun, U> m;
+  m.load(a, p, e - 1);
+  R x[U];
+  for (; e - p >= U; p += U) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      x[u] = load_row_raw<DT, V, kOff32>(a.B, m.c[u], a.ldb, col);
+    const RbEntries<DT, kRun, U> w = m;
+    m.load(a, kRun ? p + U : min(p + U, e - 1), e - 1);
+#pragma unroll
+    for (int u = 0; u < U; ++u) rb_add<DT, V, kComp>(x[u], w.val(a, u), acc, cmp);
+  }
+  if (p < e) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      x[u] = load_row_raw<DT, V, kOff32>(a.B, u < e - p ? m.c[u] : m.c[0], a.ldb, col);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      rb_add_if<DT, V, kComp>(u < e - p, x[u], m.val(a, u), acc, cmp);
+  }
+  if constexpr (kComp) {
+#pragma unroll
+    for (int j = 0; j < V; ++j) acc[j] += cmp[j];
+  }
+}
+
+// One output row of rb_sr (entries p .. e - 1) for this lane's V columns.
+template <int DT, int V, bool kOff32, int U, bool kRun>
+__device__ __forceinline__ void rb_sr_row(const KArgs &a, int32_t row, int32_t p, int32_t e,
+                                          int32_t col) {
+  float acc[V];
+  zero_vec(acc);
+  if (e - p > a.comp_threshold)
+    rb_sr_sum<DT, V, kOff32, U, kRun, true>(a, p, e, col, acc);
+  else if (p < e)
+    rb_sr_sum<DT, V, kOff32, U, kRun, false>(a, p, e, col, acc);
   store_row<V>(a.C + (int64_t)row * a.ldc + col, acc);
 }
 
-// rb_sr over row block `blk`, column panel `panel`: lane group gi owns rows
-// [gi*R, gi*R + R), R = 2^lg, one after another.
-template <int DT, int V, bool kOff32>
+// The sum of the n > 0 entries p, p + 2^lg, ... of a slot of rb_pr.
+template <int DT, int V, bool kOff32, bool kComp>
+__device__ __forceinline__ void rb_pr_sum(const KArgs &a, int32_t p, int32_t n, int lg,
+                                          int32_t col, float (&acc)[V]) {
+  using R = typename RawT<DT, V>::type;
+  constexpr int U = 4;
+  float cmp[V], v[U];
+  zero_vec(cmp);
+  const int32_t last = p + ((n - 1) << lg);
+  int32_t c[U];
+  auto entries = [&](int32_t b) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int32_t i = b + u < n ? p + ((b + u) << lg) : last;
+      c[u] = a.crd[i];
+      v[u] = load_val<DT>(a.vals, i);
+    }
+  };
+  entries(0);
+  R x[U];
+  int32_t b = 0;
+  for (; b + U <= n; b += U) {
+    float w[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      x[u] = load_row_raw<DT, V, kOff32>(a.B, c[u], a.ldb, col);
+      w[u] = v[u];
+    }
+    entries(b + U);
+#pragma unroll
+    for (int u = 0; u < U; ++u) rb_add<DT, V, kComp>(x[u], w[u], acc, cmp);
+  }
+  if (b < n) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) x[u] = load_row_raw<DT, V, kOff32>(a.B, c[u], a.ldb, col);
+#pragma unroll
+    for (int u = 0; u < U; ++u) rb_add_if<DT, V, kComp>(b + u < n, x[u], v[u], acc, cmp);
+  }
+  if constexpr (kComp) {
+#pragma unroll
+    for (int j = 0; j < V; ++j) acc[j] += cmp[j];
+  }
+}
+
+// rb_sr over row block `blk`, column panel `panel`: lane group gi owns row gi.
+template <int DT, int V, int U, bool kOff32>
 __device__ __forceinline__ void rb_sr_walk(const KArgs &a, int32_t blk,
                                            int32_t panel) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int lq = a.lq;
-  const int32_t gi =
-      ((blk * kWavesPerBlock + wave) << (6 - lq)) + (lane >> lq);
+  const int64_t row =
+      ((int64_t)(blk * kWavesPerBlock + wave) << (6 - lq)) + (lane >> lq);
   const int32_t nominal = ((panel << lq) + (lane & ((1 << lq) - 1))) * V;
-  if (nominal >= a.N) return;
   const int32_t col = lane_col<V>(nominal, a.N);
-  const int64_t first = (int64_t)gi << a.lg;
-  const int32_t R = 1 << a.lg;
-  for (int32_t i = 0; i < R; ++i) {
-    const int64_t row = first + i;
-    if (row >= a.M) return;
-    rb_sr_row<DT, V, kOff32>(a, (int32_t)row, col);
-  }
+  const bool live = row < a.M && nominal < a.N;
+  const int32_t p = live ? a.pos[row] : 0, e = live ? a.pos[row + 1] : 0;
+  // the wave's loads stay inside crd and vals, but for the last entries
+  const bool run = __ballot(live && a.nnz - e < 2 * U) == 0;
+  if (!live) return;
+  if (run)
+    rb_sr_row<DT, V, kOff32, U, true>(a, (int32_t)row, p, e, col);
+  else
+    rb_sr_row<DT, V, kOff32, U, false>(a, (int32_t)row, p, e, col);
 }
 
-template <int DT, int V>
+template <int DT, int V, int U = 8>
 __device__ __forceinline__ void rb_sr_body(const KArgs &a, int32_t blk,
                                            int32_t panel) {
   if (a.b_off32)
-    rb_sr_walk<DT, V, true>(a, blk, panel);
+    rb_sr_walk<DT, V, U, true>(a, blk, panel);
   else
-    rb_sr_walk<DT, V, false>(a, blk, panel);
+    rb_sr_walk<DT, V, U, false>(a, blk, panel);
 }
 
-// rb_pr over row block `blk`, column panel `panel`.
-template <int DT, int V, bool kOff32>
+// rb_pr over row block `blk`, column panel `panel`: R sets of 64/(P*Q) rows per
+// wave. A row of up to P entries is one step (row pointer, column, gather) of
+// three dependent loads, so a wave with several sets has them in flight
+// together.
+template <int DT, int V, bool kOff32, int R>
 __device__ __forceinline__ void rb_pr_walk(const KArgs &a, int32_t blk,
                                            int32_t panel) {
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lq = a.lq, lg = a.lg;
-  const int lr = 6 - lq - lg;  // log2(rows per wave)
-  const int32_t row0 = (blk * kWavesPerBlock + wave) << lr;
+  const int lr = 6 - lq - lg;  // log2(rows per set)
+  const int64_t row0 = ((int64_t)blk * kWavesPerBlock + wave) * R << lr;
   if (row0 >= a.M) return;  // uniform over the wave
-  const int32_t row = row0 + (lane >> (lq + lg));
   const int32_t slot = (lane >> lq) & ((1 << lg) - 1);
   const int32_t P = 1 << lg;
   const int32_t nominal = ((panel << lq) + (lane & ((1 << lq) - 1))) * V;
   const int32_t col = lane_col<V>(nominal, a.N);
-  const bool live = row < a.M && nominal < a.N;
+  const bool colok = nominal < a.N;
 
-  float acc[V];
-  zero_vec(acc);
-  if (live) {
-    const int32_t *__restrict__ crd = a.crd;
-    const void *__restrict__ vals = a.vals;
-    const void *__restrict__ B = a.B;
-    const int64_t ldb = a.ldb;
-    const int32_t s = a.pos[row];
-    const int32_t e = a.pos[row + 1];
-    int32_t p = s + slot;
-    if (e - s > a.comp_threshold) {
-      float cmp[V];
-      zero_vec(cmp);
-      for (; p < e; p += P) {
-        float b[V];
-        const float v = load_val<DT>(vals, p);
-        load_row_vec<DT, V, kOff32>(B, crd[p], ldb, col, b);
+  // this slot's entries of set k's row: p, p + P, ... (n of them)
+  int32_t p[R], n[R];
+  bool comp[R];
 #pragma unroll
-        for (int j = 0; j < V; ++j) neumaier_add(acc[j], cmp[j], v, b[j]);
+  for (int k = 0; k < R; ++k) {
+    const int64_t row = row0 + ((int64_t)k << lr) + (lane >> (lq + lg));
+    const bool live = row < a.M && colok;
+    const int32_t s = live ? a.pos[row] : 0;
+    const int32_t len = live ? a.pos[row + 1] - s : 0;
+    p[k] = s + slot;
+    n[k] = len > slot ? ((len - slot - 1) >> lg) + 1 : 0;
+    comp[k] = len > a.comp_threshold;
+  }
+  float acc[R][V];
+#pragma unroll
+  for (int k = 0; k < R; ++k) zero_vec(acc[k]);
+  if (R > 1 || __ballot(n[0] > 1) == 0) {
+    // each slot's first entry, all sets' loads in flight together (a slot
+    // without one reads entry 0)
+    if (a.nnz > 0) {
+      int32_t c[R];
+      float v[R];
+      typename RawT<DT, V>::type x[R];
+#pragma unroll
+      for (int k = 0; k < R; ++k) {
+        const int32_t i = n[k] > 0 ? p[k] : 0;
+        c[k] = a.crd[i];
+        v[k] = load_val<DT>(a.vals, i);
       }
 #pragma unroll
-      for (int j = 0; j < V; ++j) acc[j] += cmp[j];
-    } else {
-      constexpr int U = (V >= 8) ? 2 : 4;
-      for (; p + (U - 1) * P < e; p += U * P) {
-        int32_t c[U];
-        float v[U];
-        float b[U][V];
+      for (int k = 0; k < R; ++k) x[k] = load_row_raw<DT, V, kOff32>(a.B, c[k], a.ldb, col);
 #pragma unroll
-        for (int u = 0; u < U; ++u) c[u] = crd[p + u * P];
-#pragma unroll
-        for (int u = 0; u < U; ++u) v[u] = load_val<DT>(vals, p + u * P);
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-          load_row_vec<DT, V, kOff32>(B, c[u], ldb, col, b[u]);
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-          for (int j = 0; j < V; ++j) acc[j] = fmaf(v[u], b[u][j], acc[j]);
-      }
-      for (; p < e; p += P) {
-        float b[V];
-        const float v = load_val<DT>(vals, p);
-        load_row_vec<DT, V, kOff32>(B, crd[p], ldb, col, b);
-#pragma unroll
-        for (int j = 0; j < V; ++j) acc[j] = fmaf(v, b[j], acc[j]);
+      for (int k = 0; k < R; ++k) {
+        float cmp[V];
+        rb_add_if<DT, V, false>(n[k] > 0, x[k], v[k], acc[k], cmp);
       }
     }
-  }
-  // Butterfly over the P slots of each row (lane distances Q .. Q*P/2).
-  for (int d = P >> 1; d >= 1; d >>= 1) {
 #pragma unroll
-    for (int j = 0; j < V; ++j) acc[j] += __shfl_xor(acc[j], d << lq, 64);
+    for (int k = 0; k < R; ++k) {
+      if (n[k] > 0 && comp[k]) {
+        zero_vec(acc[k]);
+        rb_pr_sum<DT, V, kOff32, true>(a, p[k], n[k], lg, col, acc[k]);
+      } else if (n[k] > 1) {
+        rb_pr_sum<DT, V, kOff32, false>(a, p[k] + P, n[k] - 1, lg, col, acc[k]);
+      }
+    }
+  } else if (n[0] > 0) {
+    if (comp[0])
+      rb_pr_sum<DT, V, kOff32, true>(a, p[0], n[0], lg, col, acc[0]);
+    else
+      rb_pr_sum<DT, V, kOff32, false>(a, p[0], n[0], lg, col, acc[0]);
   }
-  if (live && slot == 0) store_row<V>(a.C + (int64_t)row * a.ldc + col, acc);
+  // butterfly over the P slots of each row (lane distances Q*P/2 .. Q)
+#pragma unroll
+  for (int k = 0; k < R; ++k) butterfly<V>(acc[k], P << lq >> 1, 1 << lq);
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const int64_t row = row0 + ((int64_t)k << lr) + (lane >> (lq + lg));
+    if (row < a.M && colok && slot == 0) store_row<V>(a.C + row * a.ldc + col, acc[k]);
+  }
 }
 
-template <int DT, int V>
+template <int DT, int V, int R = 1>
 __device__ __forceinline__ void rb_pr_body(const KArgs &a, int32_t blk,
                                            int32_t panel) {
   if (a.b_off32)
-    rb_pr_walk<DT, V, true>(a, blk, panel);
+    rb_pr_walk<DT, V, true, R>(a, blk, panel);
   else
-    rb_pr_walk<DT, V, false>(a, blk, panel);
+    rb_pr_walk<DT, V, false, R>(a, blk, panel);
 }
 
 }  // namespace segtaco
