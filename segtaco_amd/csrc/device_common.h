@@ -194,6 +194,31 @@ __device__ __forceinline__ typename RawT<DT, V>::type load_row_raw(
   }
 }
 
+// The byte offset of row `row`, and V elements from column c of the row at
+// such an offset: load_row_raw<DT, V, true> in two halves, for offsets that
+// several lanes use.
+template <int DT>
+__device__ __forceinline__ uint32_t row_offset(int32_t row, int64_t ld) {
+  return __umul24((uint32_t)row, (uint32_t)ld) * (DT == 0 ? 4 : 2);
+}
+template <int DT, int V>
+__device__ __forceinline__ typename RawT<DT, V>::type load_off_raw(
+    const void *__restrict__ base, uint32_t off, int32_t c) {
+  constexpr uint32_t kEb = DT == 0 ? 4 : 2;
+  typename RawT<DT, V>::type x;
+  __builtin_memcpy(&x, __builtin_assume_aligned(
+                           static_cast<const char *>(base) + (off + (uint32_t)c * kEb), kEb),
+                   sizeof(x));
+  return x;
+}
+
+// n elements of LDS from p (16-byte aligned), in 16-byte reads.
+template <int n, typename T>
+__device__ __forceinline__ void load_lds(const T *p, T (&x)[n]) {
+  static_assert(sizeof(T) == 4 && n % 4 == 0, "16-byte reads");
+  __builtin_memcpy(x, __builtin_assume_aligned(p, 16), sizeof(x));
+}
+
 template <int DT, int V, bool kOff32>
 __device__ __forceinline__ void load_row_vec(const void *__restrict__ base,
                                              int32_t row, int64_t ld, int32_t c,

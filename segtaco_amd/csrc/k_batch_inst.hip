@@ -72,17 +72,16 @@ __device__ __forceinline__ void dispatch(int32_t sched, int32_t vec,
 //
 // eb_sr alone fits 5 waves (96 VGPRs) without spills. 24 power-law products
 // of up to 200000 rows, FP32, N <= 128, us per launch: beside the other bodies
-// 2494, alone at 4 waves 2437, at 5 2320; 12 of up to 20000 rows, BF16, N <= 128
-// 115 / 110 / 107 (FP32 113 / 110 / 114). What bounds it is instruction issue
-// and the latency of its gathers: a wave's two lane groups end rows at different
-// steps.
+// 2494, alone at 4 waves 2437, at 5 2320, and 2202 in short batches (sched_eb.h);
+// 12 of up to 20000 rows, BF16, N <= 128 115 / 110 / 107 / 97 (FP32 113 / 110 / 114 /
+// 110). What bounds it is instruction issue and the latency of its gathers.
 template <int DT, BatchForm kForm>
 __global__ __launch_bounds__(kBlockThreads)
 __attribute__((amdgpu_waves_per_eu(kForm == kBatchEbSr ? 5 : 4))) void k_batch_main(
     const BatchDesc *__restrict__ d, int32_t n,
     const int64_t *__restrict__ prefix, int64_t total,
     unsigned long long *counter) {
-  extern __shared__ int32_t smem[];
+  extern __shared__ __align__(16) int32_t smem[];
   __shared__ int64_t s_unit;
   __shared__ int32_t s_prod;
   for (;;) {

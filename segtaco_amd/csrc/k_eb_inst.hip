@@ -11,7 +11,7 @@ namespace segtaco {
 
 template <int DT, int V>
 __global__ __launch_bounds__(kBlockThreads) void k_eb_sr(const KArgs a) {
-  extern __shared__ int32_t smem[];
+  extern __shared__ __align__(16) int32_t smem[];
   int32_t blk, panel;
   if (!decode_block(a.panels, a.nblocks, blk, panel)) return;
   eb_sr_body<DT, V>(a, blk, panel, smem);
@@ -19,7 +19,7 @@ __global__ __launch_bounds__(kBlockThreads) void k_eb_sr(const KArgs a) {
 
 template <int DT, int V>
 __global__ __launch_bounds__(kBlockThreads) void k_eb_pr(const KArgs a) {
-  extern __shared__ int32_t smem[];
+  extern __shared__ __align__(16) int32_t smem[];
   int32_t blk, panel;
   if (!decode_block(a.panels, a.nblocks, blk, panel)) return;
   eb_pr_body<DT, V>(a, blk, panel, smem);

@@ -50,11 +50,15 @@ namespace segtaco {
 
 constexpr int32_t kPosSlack = 8;   // extra pos entries staged past a chunk
 constexpr int32_t kSrChunkMax = 128;
-#ifndef SEGTACO_SR_BATCH
-#define SEGTACO_SR_BATCH 8
-#endif
-// eb_sr gathers per batch (two batches in flight per lane group)
-constexpr int kSrBatch = SEGTACO_SR_BATCH;
+// eb_sr gathers per batch (two batches in flight per lane group). What bounds
+// the walk where B stays in the caches is instruction issue: a batch in which no
+// row of the wave ends runs unrolled, and short batches are more often such ones
+// and leave registers for more waves (FP32, 4 columns: 128 -> 89). Power-law,
+// tile 128, us per call, entry by entry in batches of 8 / so with 8 / so with 4:
+// 60013^2 N = 64 BF16 61 / 46 / 43, FP32 68 / 69 / 64; 8000^2 N = 256 BF16 40 / 30 /
+// 30, FP32 37 / 31 / 30; 262144^2 N = 64 BF16 123 / 113 / 114. 24 products of up to
+// 200000 rows in a batch, FP32, N <= 128: 2328 / 2592 (spills) / 2202.
+constexpr int kSrBatch = 4;
 constexpr int32_t kPrChunk = 128;
 constexpr int kPrPasses = 8;       // eb_pr passes whose gathers are in flight
 
@@ -181,9 +185,13 @@ __device__ __forceinline__ void eb_sr_walk(const KArgs &a, int32_t blk,
       // the tile's entries are read once: non-temporal (power-law 262144^2,
       // N = 128, FP32, with the C stores above: 343 vs 352 us per step on one
       // host, the same time within 1 % on others)
-      for (int32_t i = q; i < cn; i += Q) {
-        s_crd[i] = __builtin_nontemporal_load(crd + cs + i);
-        s_val[i] = load_val_stream<DT>(vals, cs + i);
+      // (up to whole pairs of batches, with copies of its last entry)
+      const int32_t cp = (cn + 2 * kSrBatch - 1) / (2 * kSrBatch) * (2 * kSrBatch);
+      for (int32_t i = q; i < cp; i += Q) {
+        const int32_t p = cs + min(i, cn - 1);
+        const int32_t k = __builtin_nontemporal_load(crd + p);
+        s_crd[i] = kOff32 ? (int32_t)row_offset<DT>(k, ldb) : k;
+        s_val[i] = load_val_stream<DT>(vals, p);
       }
       rbase = r;
       pw = min(PW, a.M + 1 - rbase);
@@ -205,31 +213,59 @@ __device__ __forceinline__ void eb_sr_walk(const KArgs &a, int32_t blk,
       // only covers that batch and leaves the next one in flight.
       R ra[kSrBatch], rb[kSrBatch];
       auto issue = [&](R (&buf)[kSrBatch], int32_t b0) {
+        int32_t k[kSrBatch];
+        load_lds<kSrBatch>(s_crd + b0, k);
 #pragma unroll
         for (int u = 0; u < kSrBatch; ++u) {
-          const int32_t i = min(b0 + u, cn - 1);
-          buf[u] = load_row_raw<DT, V, kOff32>(B, s_crd[i], ldb, col);
+          if constexpr (kOff32)
+            buf[u] = load_off_raw<DT, V>(B, (uint32_t)k[u], col);
+          else
+            buf[u] = load_raw<DT, V>(B, (int64_t)k[u] * ldb + col);
         }
       };
+      auto add = [&](const R &x, float v) {
+        float b[V];
+        unpack<DT, V>(x, b);
+        if (comp) {
+#pragma unroll
+          for (int j = 0; j < V; ++j) neumaier_add(acc[j], cmp[j], v, b[j]);
+        } else {
+#pragma unroll
+          for (int j = 0; j < V; ++j) acc[j] = fmaf(v, b[j], acc[j]);
+        }
+      };
+      // (lanes past N sum their last columns too, and store nothing)
       auto consume = [&](const R (&buf)[kSrBatch], int32_t b0) {
         const int32_t nb = min(kSrBatch, cn - b0);
+        if (__ballot(nb < kSrBatch || re < cs + b0 + kSrBatch) == 0) {
+          // every group's row goes on to the end of the batch
+          float v[kSrBatch];
+          load_lds<kSrBatch>(s_val + b0, v);
+          if (comp) {
+#pragma unroll
+            for (int u = 0; u < kSrBatch; ++u) {
+              float b[V];
+              unpack<DT, V>(buf[u], b);
+#pragma unroll
+              for (int j = 0; j < V; ++j) neumaier_add(acc[j], cmp[j], v[u], b[j]);
+            }
+          } else {
+#pragma unroll
+            for (int u = 0; u < kSrBatch; ++u) {
+              float b[V];
+              unpack<DT, V>(buf[u], b);
+#pragma unroll
+              for (int j = 0; j < V; ++j) acc[j] = fmaf(v[u], b[j], acc[j]);
+            }
+          }
+          return;
+        }
 #pragma unroll
         for (int u = 0; u < kSrBatch; ++u) {
           if (u < nb) {
             const int32_t pp = cs + b0 + u;
             if (pp == re) next_row(pp);
-            if (colok) {
-              const float v = s_val[b0 + u];
-              float b[V];
-              unpack<DT, V>(buf[u], b);
-              if (comp) {
-#pragma unroll
-                for (int j = 0; j < V; ++j) neumaier_add(acc[j], cmp[j], v, b[j]);
-              } else {
-#pragma unroll
-                for (int j = 0; j < V; ++j) acc[j] = fmaf(v, b[j], acc[j]);
-              }
-            }
+            add(buf[u], s_val[b0 + u]);
           }
         }
       };
