@@ -6,9 +6,9 @@
 // with the K21 partition, FP64 values and one warp atomic per entry; :5-44,
 // a warp per row; both are disabled in the reference's build.)
 //
-// Here the entries are cut into tiles of kSdTile consecutive entries, one
-// wave per tile, and the tile's first row comes from the same partition pass
-// the SpMM schedules use (k_tile_rows: the repaired K21 row). Each chunk of the
+// Here the entries are cut into tiles of 16 to kSdTile consecutive entries, one
+// wave per tile, which finds the tile's rows itself (a 64-way search of pos:
+// the rows that the K21 partition would give). Each chunk of the
 // tile stages its column indices, values and a window of the row pointer in
 // LDS and resolves every entry's row by a binary search there. The wave is
 // P = 64/Q slots of Q lanes; per batch a slot takes U consecutive entries,
@@ -17,6 +17,13 @@
 // tree (transposed across the U entries, then a butterfly). Every out[p]
 // has exactly one writer and a fixed summation order: no atomics, no
 // clearing, and results are identical run to run.
+//
+// A row's J elements are taken in the widest slices whatever J and the
+// alignment (gfx950 loads 16 bytes at any element): 60013^2, J = 77, us per call
+// with one element per load / so: FP32 180 / 58, BF16 181 / 47. Large products are
+// bound by the gathered lines of Y (262144^2, J = 128, FP32: 4.2 M rows of 512
+// bytes in 318 us, 6.9 TB/s), small ones by the waves in flight and the chain of
+// index, gather and reduction.
 #include <climits>
 
 #include "device_common.h"
@@ -30,7 +37,7 @@ constexpr int32_t kSdChunk = 128;
 constexpr int32_t kSdPosSlack = 8;
 constexpr int kSdU = 4;  // consecutive entries per slot and batch
 
-template <int DT, int V, bool kOff32>
+template <int DT, int V, bool kOff32, bool kRag>
 __global__ __launch_bounds__(256) void k_sddmm(const SddmmArgs a) {
   __shared__ int32_t smem[4 * (4 * kSdChunk + kSdPosSlack)];
   const int lane = threadIdx.x & 63;
@@ -53,8 +60,9 @@ __global__ __launch_bounds__(256) void k_sddmm(const SddmmArgs a) {
   const int32_t *__restrict__ crd = a.crd;
   const int32_t s = t * a.tile;
   const int32_t e = (int32_t)min((int64_t)a.nnz, (int64_t)s + a.tile);
-  const int32_t r_hi = min(a.M - 1, a.tile_row[t + 1]);
-  int32_t r = a.tile_row[t];
+  int32_t r, r_hi;  // rows of entries s and e
+  wave_rows_of(pos, a.M, s, e, r, r_hi);
+  r_hi = min(r_hi, a.M - 1);
   using R = typename RawT<DT, V>::type;
   // With Q >= kSdU lanes per slot the kSdU partial sums of a batch are
   // reduced together (transposed); with fewer, one butterfly per entry.
@@ -103,7 +111,10 @@ __global__ __launch_bounds__(256) void k_sddmm(const SddmmArgs a) {
       for (int32_t jc = 0; jc < a.J; jc += Q * V) {
         const int32_t c = jc + q * V;
         const bool cok = c < a.J;
-        const int32_t c_ld = cok ? c : 0;
+        // kRag: the last slice is moved back to end at J, and its columns that
+        // the slice before it holds are not added
+        const int32_t c_ld = kRag ? lane_col<V>(c, a.J) : cok ? c : 0;
+        const int32_t skip = kRag ? c - c_ld : 0;
         R xr[kSdU], yr[kSdU];
 #pragma unroll
         for (int u = 0; u < kSdU; ++u) {
@@ -117,7 +128,10 @@ __global__ __launch_bounds__(256) void k_sddmm(const SddmmArgs a) {
             unpack<DT, V>(xr[u], x);
             unpack<DT, V>(yr[u], y);
 #pragma unroll
-            for (int j = 0; j < V; ++j) part[u] = fmaf(x[j], y[j], part[u]);
+            for (int j = 0; j < V; ++j) {
+              const float f = fmaf(x[j], y[j], part[u]);
+              part[u] = !kRag || j >= skip ? f : part[u];
+            }
           }
         }
       }
@@ -157,18 +171,22 @@ __global__ __launch_bounds__(256) void k_sddmm(const SddmmArgs a) {
 
 }  // namespace
 
-int32_t sddmm_tile() { return kSdTile; }
-
 hipError_t launch_sddmm(int dt, int vec, const SddmmArgs &a, hipStream_t s) {
   const int64_t grid = (a.ntiles + 3) / 4;
   if (grid <= 0) return hipSuccess;
   const dim3 g((unsigned)grid), b(256);
 #define SEGTACO_SD_CASE(DT, V)                                                  \
   case DT * 16 + V:                                                             \
-    if (a.off32)                                                                \
-      hipLaunchKernelGGL((k_sddmm<DT, V, true>), g, b, 0, s, a);                \
-    else                                                                        \
-      hipLaunchKernelGGL((k_sddmm<DT, V, false>), g, b, 0, s, a);               \
+    if (V > 1 && a.J % V) {                                                     \
+      if (a.off32)                                                              \
+        hipLaunchKernelGGL((k_sddmm<DT, V, true, (V > 1)>), g, b, 0, s, a);     \
+      else                                                                      \
+        hipLaunchKernelGGL((k_sddmm<DT, V, false, (V > 1)>), g, b, 0, s, a);    \
+    } else if (a.off32) {                                                       \
+      hipLaunchKernelGGL((k_sddmm<DT, V, true, false>), g, b, 0, s, a);         \
+    } else {                                                                    \
+      hipLaunchKernelGGL((k_sddmm<DT, V, false, false>), g, b, 0, s, a);        \
+    }                                                                           \
     break;
   switch (dt * 16 + vec) {
     SEGTACO_SD_CASE(0, 1)

@@ -53,45 +53,6 @@ constexpr uint32_t kSegComp = 0x8000;   // of a compensated row
 constexpr uint32_t kSegMany = 0x4000;   // of a segment over several tiles
 constexpr uint32_t kSegFirst = 0x2000;  // the segment's first piece
 
-// Last row r in [lo, hi) with pos[r] <= target, given pos[lo] <= target <
-// pos[hi]: 64 probes per step. The whole wave calls it; the result is uniform.
-__device__ __forceinline__ int32_t wave_row_of(const int32_t *__restrict__ pos, int32_t lo,
-                                               int32_t hi, int32_t target) {
-  const int32_t lane = threadIdx.x & 63;
-  while (hi - lo > 1) {
-    const int32_t step = ((hi - lo - 1) >> 6) + 1;
-    const int64_t at = (int64_t)lo + (int64_t)(lane + 1) * step;
-    const bool le = at < hi && pos[at] <= target;
-    const int32_t c = __popcll(__ballot(le));  // probes are ascending
-    lo += c * step;
-    hi = (int32_t)min((int64_t)hi, (int64_t)lo + step);
-  }
-  return lo;
-}
-
-// Two wave_row_of searches in [0, M) at once (their probe loads overlap):
-// the rows of entries e0 and e1 (e1 >= nnz: M).
-__device__ __forceinline__ void wave_rows_of(const int32_t *__restrict__ pos, int32_t M,
-                                             int32_t e0, int32_t e1, int32_t &r0, int32_t &r1) {
-  const int32_t lane = threadIdx.x & 63;
-  int32_t l0 = 0, l1 = 0, h0 = M, h1 = M;
-  while (h0 - l0 > 1 || h1 - l1 > 1) {
-    const int32_t st0 = ((h0 - l0 - 1) >> 6) + 1, st1 = ((h1 - l1 - 1) >> 6) + 1;
-    const int64_t a0 = (int64_t)l0 + (int64_t)(lane + 1) * st0;
-    const int64_t a1 = (int64_t)l1 + (int64_t)(lane + 1) * st1;
-    // clamped probes load pos[M] (= nnz, above e0); no branch around the loads
-    const int32_t p0 = pos[a0 < h0 ? a0 : M], p1 = pos[a1 < h1 ? a1 : M];
-    const int32_t c0 = __popcll(__ballot(a0 < h0 && p0 <= e0));
-    const int32_t c1 = __popcll(__ballot(a1 < h1 && p1 <= e1));
-    l0 += c0 * st0;
-    l1 += c1 * st1;
-    h0 = (int32_t)min((int64_t)h0, (int64_t)l0 + st0);
-    h1 = (int32_t)min((int64_t)h1, (int64_t)l1 + st1);
-  }
-  r0 = l0;
-  r1 = l1;
-}
-
 template <int DT, int V, bool kOff32, bool kComp>
 __global__ __launch_bounds__(64) void k_eb_seg(const SegArgs g) {
   extern __shared__ __align__(16) char smem[];

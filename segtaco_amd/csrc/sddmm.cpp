@@ -1,6 +1,9 @@
 // sddmm.cpp — host side of the SDDMM entry point (include/segtaco/sddmm.h):
-// operand checks, vector width / lane count selection, the shared row
-// partition pass, and the kernel launch.
+// operand checks, vector width, lane count and tile selection, and the kernel
+// launch. The kernel finds its rows itself; the workspace that the entry point
+// asks for is left untouched.
+#include <algorithm>
+
 #include "engine.h"
 #include "launch.h"
 #include "sddmm.h"
@@ -9,12 +12,22 @@
 namespace segtaco {
 namespace {
 
-int64_t sddmm_tiles(const segtaco_csr_t *S) {
-  return S->nnz > 0 ? ceil_div(S->nnz, kSdTile) : 0;
-}
-
-bool aligned(const void *p, int64_t bytes) {
-  return (reinterpret_cast<uintptr_t>(p) % (uintptr_t)bytes) == 0;
+// Entries per wave: as few as give 4096 waves (four per SIMD), but 16 and about
+// a batch of the wave's slots at least; where 512 entries per wave are more
+// waves than the chip holds (about 7000) and an entry is work enough, short
+// tiles again. Power-law, us per call at the tiles 512 / 256 / 128 / 64 / 32 / 16
+// (before, with a partition launch and tiles of 512):
+//   1000^2 (16 K entries) J = 128 FP32 57 / 29 / 16 / 9.3 / 6.4 / 5.0 (58), J = 8 13 /
+//     7.7 / 5.0 / 4.4 / 4.4 / 4.4 (15)
+//   8000^2 (125 K) J = 128 FP32 71 / 37 / 21 / 13 / 11 / 14 (72), J = 8 14 / 8.3 / 5.6 /
+//     5.1 / 5.7 / 8.9 (16)
+//   60013^2 (960 K) J = 16 FP32 23 / 17 / 18 (24), J = 128 BF16 49 / 38 / 38 (51)
+//   262144^2 (4.2 M) J = 128 FP32 340 / 326 / 318 (341), J = 8 BF16 54 / 57 / 62 (53)
+int32_t sddmm_tile(int64_t nnz, int64_t row_bytes, int32_t lq) {
+  if (nnz >= 3584 * 1024 && row_bytes >= 128) return 128;
+  int32_t tile = std::max(16, std::min(64, 256 >> lq));
+  while (tile < kSdTile && nnz > (int64_t)4096 * tile) tile <<= 1;
+  return tile;
 }
 
 }  // namespace
@@ -26,7 +39,7 @@ extern "C" {
 
 size_t segtaco_sddmm_workspace_bytes(const segtaco_csr_t *S) {
   if (!S || S->nnz <= 0) return 0;
-  return align_up(sizeof(int32_t) * (size_t)(sddmm_tiles(S) + 1), 256);
+  return align_up(sizeof(int32_t) * (size_t)(ceil_div(S->nnz, kSdTile) + 1), 256);
 }
 
 int32_t segtaco_sddmm(const segtaco_csr_t *S, const void *X, int64_t ldx,
@@ -58,12 +71,9 @@ int32_t segtaco_sddmm(const segtaco_csr_t *S, const void *X, int64_t ldx,
   if (!workspace || workspace_bytes < need)
     return set_error(SEGTACO_ERR_INVALID, "segtaco_sddmm: workspace of %zu bytes needed",
                      need);
-  // widest vector that J, both leading dimensions and both bases allow
   const int32_t eb = elem_bytes(dtype);
   int32_t V = dtype == SEGTACO_DT_F32 ? 4 : 8;
-  while (V > 1 && (J % V || ldx % V || ldy % V || !aligned(X, (int64_t)V * eb) ||
-                   !aligned(Y, (int64_t)V * eb)))
-    V >>= 1;
+  while (V > J) V >>= 1;
   int32_t lq = 0;
   while ((1 << lq) < 64 && (int64_t)(1 << lq) * V < J) ++lq;
 
@@ -82,11 +92,8 @@ int32_t segtaco_sddmm(const segtaco_csr_t *S, const void *X, int64_t ldx,
   a.out = out;
   a.lq = lq;
   a.off32 = b_off32_ok(S->M, ldx, eb) && b_off32_ok(S->K, ldy, eb);
-  a.tile = kSdTile;
-  a.ntiles = (int32_t)sddmm_tiles(S);
-  int32_t *tile_row = static_cast<int32_t *>(workspace);
-  a.tile_row = tile_row;
-  SEGTACO_HIP(launch_tile_rows(S->pos, S->M, kSdTile, a.ntiles, tile_row, stream));
+  a.tile = sddmm_tile(S->nnz, (int64_t)J * eb, lq);
+  a.ntiles = (int32_t)ceil_div(S->nnz, a.tile);
   SEGTACO_HIP(launch_sddmm(dtype, V, a, stream));
   return SEGTACO_OK;
 }

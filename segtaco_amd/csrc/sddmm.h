@@ -7,7 +7,7 @@
 
 namespace segtaco {
 
-constexpr int32_t kSdTile = 512;  // entries per wave (one tile)
+constexpr int32_t kSdTile = 512;  // entries per wave (one tile) at most
 
 struct SddmmArgs {
   int32_t M, K, J, nnz;
@@ -20,15 +20,13 @@ struct SddmmArgs {
   int64_t ldy;
   float *out;        // nnz
   int32_t lq;        // log2(lanes per entry)
-  int32_t tile;      // entries per tile (kSdTile)
+  int32_t tile;      // entries per wave (one tile)
   int32_t ntiles;
-  const int32_t *tile_row;  // row holding each tile's first entry (ntiles+1)
   // row * ld + column (elements) of X and Y fits 32 bits after scaling to
   // bytes, and every row index and leading dimension is below 2^24
   int32_t off32;
 };
 
-int32_t sddmm_tile();
 hipError_t launch_sddmm(int dt, int vec, const SddmmArgs &a, hipStream_t s);
 
 }  // namespace segtaco
