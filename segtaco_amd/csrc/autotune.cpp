@@ -274,24 +274,38 @@ int32_t segtaco_tune_measure(const segtaco_csr_t *A,
   float best = 1e30f, best_shared = 1e30f;
   segtaco_plan_t best_plan = model, shared_plan = model;
   int32_t status = SEGTACO_OK;
-  for (const auto &p : plans) {
-    status = spmm_impl(A, B, b_dtype, ldb, N, C, ldc, &p, ws, ws_need, stream, nullptr);
-    if (status != SEGTACO_OK) break;
-    if (hipEventRecord(e0, stream) != hipSuccess) { status = SEGTACO_ERR_HIP; break; }
-    for (int32_t r = 0; r < reps && status == SEGTACO_OK; ++r)
-      status = spmm_impl(A, B, b_dtype, ldb, N, C, ldc, &p, ws, ws_need, stream, nullptr);
-    if (status != SEGTACO_OK) break;
+  auto time_plan = [&](const segtaco_plan_t &p, int32_t phases, float *ms) -> int32_t {
+    SEGTACO_RET(spmm_impl(A, B, b_dtype, ldb, N, C, ldc, &p, ws, ws_need, stream, nullptr,
+                          phases));
+    if (hipEventRecord(e0, stream) != hipSuccess) return SEGTACO_ERR_HIP;
+    for (int32_t r = 0; r < reps; ++r)
+      SEGTACO_RET(spmm_impl(A, B, b_dtype, ldb, N, C, ldc, &p, ws, ws_need, stream, nullptr,
+                            phases));
     if (hipEventRecord(e1, stream) != hipSuccess ||
-        hipEventSynchronize(e1) != hipSuccess) {
-      status = SEGTACO_ERR_HIP;
-      break;
-    }
+        hipEventSynchronize(e1) != hipSuccess)
+      return SEGTACO_ERR_HIP;
+    *ms = 0.f;
+    (void)hipEventElapsedTime(ms, e0, e1);
+    *ms /= reps;
+    return SEGTACO_OK;
+  };
+  for (const auto &p : plans) {
     float ms = 0.f;
-    (void)hipEventElapsedTime(&ms, e0, e1);
-    ms /= reps;
+    status = time_plan(p, kPhaseAll, &ms);
+    if (status != SEGTACO_OK) break;
     if (ms < best) {
       best = ms;
       best_plan = p;
+    }
+    // The plan that batches share is chosen by the kernel that a batch runs: a
+    // single eb_sr call of up to 64 columns may take the segment form, which a
+    // batch does not have and whose time hardly depends on the tile (512
+    // power-law products, FP32, N in {16, 32, 64, 128}, ms per launch: 90.6 and
+    // 102.7 in two tunings by the single calls' times, 87.9 to 90.8 in three by
+    // the walk's).
+    if (p.schedule == SEGTACO_EB_SR && N <= 64) {
+      status = time_plan(p, kPhaseAll | kPhaseWalk, &ms);
+      if (status != SEGTACO_OK) break;
     }
     if (shared_schedule(p.schedule) && ms < best_shared) {
       best_shared = ms;

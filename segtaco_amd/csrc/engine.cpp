@@ -536,7 +536,7 @@ int32_t spmm_impl(const segtaco_csr_t *A, const void *B, int32_t b_dtype,
                   hipStream_t stream, hipEvent_t *ev, int32_t phases) {
   SEGTACO_RET(check_csr(A));
   if (!plan_in) return set_error(SEGTACO_ERR_INVALID, "null plan");
-  if (phases < kPhasePrepare || phases > kPhaseAll)
+  if (phases < kPhasePrepare || phases > (kPhaseAll | kPhaseWalk))
     return set_error(SEGTACO_ERR_INVALID, "phases %d", phases);
   const bool prepare = (phases & kPhasePrepare) != 0;
   const bool run = (phases & kPhaseRun) != 0;
@@ -711,7 +711,7 @@ int32_t spmm_impl(const segtaco_csr_t *A, const void *B, int32_t b_dtype,
   if (prepare) prep_record(ws, nullptr);
   SEGTACO_HIP(mark(0));
   const int64_t tiles_per_block = (int64_t)kWavesPerBlock * (64 / form.lanes);
-  if (run && plan.schedule == SEGTACO_EB_SR) {
+  if (run && !(phases & kPhaseWalk) && plan.schedule == SEGTACO_EB_SR) {
     SegArgs g;
     if (const int32_t sv =
             seg_plan(b_dtype, a, ceil_div(L.ntiles, tiles_per_block) * a.panels, &g)) {

@@ -66,6 +66,8 @@ int32_t device_cus();
 constexpr int32_t kPhasePrepare = 1;
 constexpr int32_t kPhaseRun = 2;
 constexpr int32_t kPhaseAll = kPhasePrepare | kPhaseRun;
+// Beside kPhaseAll: eb_sr as a batch runs it, never in the segment form.
+constexpr int32_t kPhaseWalk = 4;
 
 // The device API's implementation (engine.cpp). ev: 4 optional events
 // recorded around partition, main kernel and fix-up. phases: kPhaseAll for
