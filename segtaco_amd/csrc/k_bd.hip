@@ -327,9 +327,9 @@ __device__ bool bd_mfma(const KArgs &a, BdShared<CT, RB> &sh, const int32_t *pos
   } else {
     // 256-column panels go through LDS, 16 rows at a time, so that a wave
     // stores a row's 1 KB with 16-byte stores instead of 128-byte pieces of two
-    // rows (banded BF16, direct / so: 1M^2 N = 256 467 / 419 us per call, where
-    // copies reach this kernel's 2.0 GB in 424 us; 400000^2 N = 200 224 / 158;
-    // panels of 128 columns 291 / 295)
+    // rows (banded BF16, before / so, us per call: 400000^2 N = 200 196 / 157;
+    // 1M^2 N = 256, where copies reach this kernel's 2.0 GB in 408 us, 418 / 415;
+    // panels of 128 columns 291 / 295, so they store directly)
     constexpr int32_t kCStride = kCols + 4;
     float *sc = reinterpret_cast<float *>(sh.A);  // over A and B, both consumed
     static_assert(sizeof(sh.A) + sizeof(sh.B) >= 16 * kCStride * sizeof(float),
