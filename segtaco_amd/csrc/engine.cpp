@@ -312,6 +312,16 @@ int32_t check_csr(const segtaco_csr_t *A) {
   return SEGTACO_OK;
 }
 
+// Columns per lane of an eb_cs plan, whose LDS slots hold kCsLanes * vec
+// floats: at most 4, and at least the plan's. The workspace is laid out by it,
+// also for plans whose fields no call would accept (a vec below 1 stays).
+int32_t cs_vec(const segtaco_plan_t &p, int32_t N, int32_t b_dtype) {
+  const int32_t w = widest_any(b_dtype, N);
+  int32_t v = p.vec;
+  while (v > 0 && v < w && v < 4 && kCsLanes * v < N) v <<= 1;
+  return v;
+}
+
 }  // namespace
 
 // The vector width and lanes a resolved plan runs with; no choice here changes
@@ -370,8 +380,9 @@ ExecForm exec_form(const segtaco_plan_t &p, int32_t M, int32_t nnz, int32_t N,
       while (f.vec < w && f.lanes * f.vec < N) f.vec <<= 1;
       items = ceil_div(nnz, p.tile) * p.group;
       break;
-    case SEGTACO_EB_CS:  // LDS slots of lanes * vec floats, vec at most 4
-      while (f.vec < w && f.vec < 4 && f.lanes * f.vec < N) f.vec <<= 1;
+    case SEGTACO_EB_CS:
+      f.vec = cs_vec(p, N, b_dtype);
+      f.lanes = kCsLanes;
       items = INT64_MAX / 64;
       break;
     default:
@@ -392,9 +403,7 @@ namespace {
 size_t resolved_workspace_bytes(const segtaco_csr_t *A, int32_t N,
                                 const segtaco_plan_t &p, int32_t b_dtype) {
   if (p.schedule == SEGTACO_EB_CS)
-    return cs_layout(A->nnz, A->K, N, p.tile, p.group,
-                     exec_form(p, A->M, A->nnz, N, b_dtype).vec)
-        .total;
+    return cs_layout(A->nnz, A->K, N, p.tile, p.group, cs_vec(p, N, b_dtype)).total;
   if (p.schedule != SEGTACO_EB_SR && p.schedule != SEGTACO_EB_PR) return 0;
   return eb_layout(A->nnz, N, p.tile).total;
 }
@@ -459,7 +468,7 @@ int32_t cs_workspace_layout_impl(const segtaco_csr_t *A, int32_t N,
   if (plan->tile < 8 || plan->vec < 1 || plan->group < 1)
     return set_error(SEGTACO_ERR_INVALID, "segtaco_cs_workspace_layout: unresolved plan");
   const CsLayout L = cs_layout(A->nnz, A->K, N, plan->tile, plan->group,
-                               exec_form(*plan, A->M, A->nnz, N, SEGTACO_DT_F32).vec);
+                               cs_vec(*plan, N, SEGTACO_DT_F32));
   const int64_t v[10] = {L.units, L.cap, L.packed,
                          (int64_t)L.rec_off, (int64_t)L.rows_off, (int64_t)L.int_off,
                          (int64_t)L.code_off, (int64_t)L.nslot_off, (int64_t)L.count_off,
