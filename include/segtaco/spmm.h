@@ -209,9 +209,17 @@ void spmm_csr_gpu_cusparse(taco_tensor_t *C, taco_tensor_t *A, taco_tensor_t *B)
 typedef struct segtaco_plan {
   int32_t schedule;       /* SEGTACO_RB_SR .. SEGTACO_EB_PR */
   int32_t vec;            /* elements of B per lane per load (1,2,4; 8 for
-                             16-bit storage); 0 = widest N allows */
+                             16-bit storage), dividing N and the leading
+                             dimensions; 0 = widest they allow. A narrower
+                             value than that is kept; the widest leaves the
+                             call to take a row in other slices (odd widths
+                             in wide ones, the last moved back to end at N;
+                             eb_sr in narrower ones over more lanes), which
+                             changes no sum. eb_cs: at least this many */
   int32_t col_lanes;      /* lanes sharing one B row segment, power of two
-                             1..64; the column tile is col_lanes * vec */
+                             1..64; the column tile is col_lanes * vec. 0 =
+                             all that a row can use, up to 64 (rb_pr 16,
+                             eb_pr 32); rb_sr and eb_sr keep another value */
   int32_t group;          /* *_pr: nnz slots reduced together (power of two);
                              rb_sr: rows per lane group; 0 = auto */
   int32_t tile;           /* eb_*: nnz per tile (multiple of 8); 0 = auto:
@@ -356,6 +364,16 @@ int32_t segtaco_spmm_workspace_layout(const segtaco_csr_t *A, int32_t N,
  * row, 4 walks). */
 int32_t segtaco_cs_workspace_layout(const segtaco_csr_t *A, int32_t N,
                                     const segtaco_plan_t *plan, int64_t *out);
+
+/* The form a call of segtaco_spmm (batch = 0) or the same product in a batch
+ * (batch = 1) runs for these operands (of B and C only the alignment counts):
+ * out[0] = elements of B per lane and load, out[1] = lanes per B row segment;
+ * out[2], out[3] = for eb_sr calls in the segment form (short lane groups sum
+ * row pieces from LDS) the elements per lane of its gather and the tiles per
+ * wave, else 0. */
+int32_t segtaco_spmm_form(const segtaco_csr_t *A, const void *B, int32_t b_dtype,
+                          int64_t ldb, int32_t N, const float *C, int64_t ldc,
+                          const segtaco_plan_t *plan, int32_t batch, int32_t *out);
 
 /* rows[p] for every stored entry p < nnz: its row as the eb_pr schedule
  * derives it inside tiles of `tile` entries (per 128-entry chunk, a

@@ -203,6 +203,10 @@ def lib() -> ctypes.CDLL:
     L.segtaco_cs_workspace_layout.argtypes = [ctypes.POINTER(CSR), ctypes.c_int32,
                                               ctypes.POINTER(Plan),
                                               ctypes.POINTER(ctypes.c_int64)]
+    L.segtaco_spmm_form.restype = ctypes.c_int32
+    L.segtaco_spmm_form.argtypes = [ctypes.POINTER(CSR), _vp, ctypes.c_int32, ctypes.c_int64,
+                                    ctypes.c_int32, _vp, ctypes.c_int64,
+                                    ctypes.POINTER(Plan), ctypes.c_int32, _i32p]
     L.segtaco_entry_rows.restype = ctypes.c_int32
     L.segtaco_entry_rows.argtypes = [_vp, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, _vp,
                                      _vp, _vp]
@@ -701,6 +705,17 @@ def cs_workspace_layout(A: CSR, N: int, plan: Plan) -> dict:
     keys = ("units", "cap", "packed", "rec_off", "slot_rows_off", "int_rows_off",
             "codes_off", "n_slots_off", "tile_count_off", "tile_flags_off")
     return {k: int(v) for k, v in zip(keys, out)}
+
+
+def spmm_form(A: CSR, N: int, b_dtype: int, plan: Plan, ldb: int | None = None,
+              ldc: int | None = None, B_ptr: int = 0, C_ptr: int = 0,
+              batch: bool = False) -> dict:
+    """The slice width and lanes a call (or the product in a batch) runs with, and
+    for an eb_sr call in the segment form its gather width and tiles per wave."""
+    out = (ctypes.c_int32 * 4)()
+    check(lib().segtaco_spmm_form(ctypes.byref(A), B_ptr or None, b_dtype, ldb or N, N,
+                                  C_ptr or None, ldc or N, ctypes.byref(plan), int(batch), out))
+    return dict(vec=out[0], lanes=out[1], seg_vec=out[2], seg_tiles=out[3])
 
 
 def entry_rows(pos_ptr: int, M: int, nnz: int, T: int, tile_rows_ptr: int, rows_ptr: int,

@@ -100,7 +100,8 @@ void fill_batch_desc(const segtaco_csr_t &A, const void *B, int64_t ldb,
   a.b_off32 = b_off32_ok(A.K, ldb, 4);
   a.C = C;
   a.ldc = ldc;
-  const ExecForm form = exec_form(plan, A.M, A.nnz, N, b_dtype);
+  const ExecForm form =
+      exec_form(plan, A.M, A.nnz, N, b_dtype, widest_vec(b_dtype, N, ldb, ldc, B, C));
   a.lq = form.lq;
   a.lg = ilog2(plan.group);
   a.tile = plan.tile;

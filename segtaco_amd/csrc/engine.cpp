@@ -140,6 +140,8 @@ bool aligned(const void *p, size_t a) {
   return ((uintptr_t)p % a) == 0;
 }
 
+}  // namespace
+
 // Widest per-lane vector (in elements) that N, the leading dimensions and the
 // base pointers allow.
 int32_t widest_vec(int32_t dt, int32_t N, int64_t ldb, int64_t ldc,
@@ -153,6 +155,8 @@ int32_t widest_vec(int32_t dt, int32_t N, int64_t ldb, int64_t ldc,
   }
   return 1;
 }
+
+namespace {
 
 int32_t natural_lanes(int32_t N, int32_t vec) {
   int64_t q = pow2_ceil(ceil_div(N, vec));
@@ -327,10 +331,12 @@ int32_t cs_vec(const segtaco_plan_t &p, int32_t N, int32_t b_dtype) {
 // The vector width and lanes a resolved plan runs with; no choice here changes
 // a sum's order.
 //
-// A plan's vec divides N and the leading dimensions, so an odd width would run
-// with one element per lane and load, in several panels; the kernels take a
-// row's columns in wider slices, the last one moved back to end at N
-// (lane_col). The width is the smallest that takes the row in one panel: of
+// A plan that names a narrower slice than the operands allow, or for eb_sr and
+// rb_sr other lanes than the row spreads over, runs as it says. The rest is
+// chosen here. A plan's vec divides N and the leading dimensions, so an odd
+// width would run with one element per lane and load, in several panels; the
+// kernels take a row's columns in wider slices, the last one moved back to end
+// at N (lane_col). The width is the smallest that takes the row in one panel: of
 // the plan's lanes for the schedules whose lanes and slots fill the wave
 // (their slots stay), of half a wave for eb_sr, whose groups then share it,
 // and for rb_sr where a whole wave does not take the row. Measured at N = 77,
@@ -350,22 +356,24 @@ int32_t cs_vec(const segtaco_plan_t &p, int32_t N, int32_t b_dtype) {
 // products of 2000 to 20000 rows: BF16 N <= 64 286 / 119, FP32 N <= 64 164 / 118;
 // 24 of up to 200000 rows, FP32 N <= 128 2440 / 2320).
 ExecForm exec_form(const segtaco_plan_t &p, int32_t M, int32_t nnz, int32_t N,
-                   int32_t b_dtype) {
-  ExecForm f{p.vec, p.col_lanes, 0, 1};
+                   int32_t b_dtype, int32_t widest) {
+  ExecForm f{p.vec, p.col_lanes, 0, 1, false};
   const int32_t w = widest_any(b_dtype, N);
+  const bool open_vec = p.vec >= widest;
   // plans that spread a row over all the lanes it can use
   const bool natural = p.col_lanes == natural_lanes(N, p.vec);
+  f.own = open_vec && natural;
   int64_t items = 0;  // lane groups of the launch
   switch (p.schedule) {
     case SEGTACO_RB_SR:
-      if (natural && 64 * f.vec < N) {
+      if (f.own && 64 * f.vec < N) {
         while (f.vec < w && 32 * f.vec < N) f.vec <<= 1;
         f.lanes = natural_lanes(N, f.vec);
       }
       items = M;
       break;
     case SEGTACO_EB_SR:
-      if (natural) {
+      if (f.own) {
         f.vec = N > 16 && nnz > 1200000 ? 2 : 1;
         while (f.vec < w && f.vec < 4 && 32 * f.vec < N) f.vec <<= 1;
         f.lanes = natural_lanes(N, f.vec);
@@ -373,11 +381,13 @@ ExecForm exec_form(const segtaco_plan_t &p, int32_t M, int32_t nnz, int32_t N,
       items = ceil_div(nnz, p.tile);
       break;
     case SEGTACO_RB_PR:
-      while (f.vec < w && f.lanes * f.vec < N) f.vec <<= 1;
+      if (open_vec)
+        while (f.vec < w && f.lanes * f.vec < N) f.vec <<= 1;
       items = (int64_t)M * p.group;
       break;
     case SEGTACO_EB_PR:
-      while (f.vec < w && f.lanes * f.vec < N) f.vec <<= 1;
+      if (open_vec)
+        while (f.vec < w && f.lanes * f.vec < N) f.vec <<= 1;
       items = ceil_div(nnz, p.tile) * p.group;
       break;
     case SEGTACO_EB_CS:
@@ -497,6 +507,11 @@ struct PrepKey {
   }
 };
 
+// Workgroups of k_eb_sr's launch over ntiles tiles.
+int64_t seg_walk_blocks(const ExecForm &f, int64_t ntiles) {
+  return ceil_div(ntiles, (int64_t)kWavesPerBlock * (64 / f.lanes)) * f.panels;
+}
+
 std::mutex g_prep_mu;
 std::unordered_map<const void *, PrepKey> g_prepared;
 constexpr size_t kMaxPrepared = 4096;  // forgotten beyond: run-only calls then fail
@@ -584,7 +599,8 @@ int32_t spmm_impl(const segtaco_csr_t *A, const void *B, int32_t b_dtype,
   a.b_off32 = b_off32_ok(A->K, ldb, elem_bytes(b_dtype));
   a.C = C;
   a.ldc = ldc;
-  const ExecForm form = exec_form(plan, A->M, A->nnz, N, b_dtype);
+  const ExecForm form = exec_form(plan, A->M, A->nnz, N, b_dtype,
+                                  widest_vec(b_dtype, N, ldb, ldc, B, C));
   const int32_t V = form.vec;
   a.lq = form.lq;
   // rb_sr's rows per group only order the launch: one row per group keeps
@@ -720,10 +736,9 @@ int32_t spmm_impl(const segtaco_csr_t *A, const void *B, int32_t b_dtype,
   if (prepare) prep_record(ws, nullptr);
   SEGTACO_HIP(mark(0));
   const int64_t tiles_per_block = (int64_t)kWavesPerBlock * (64 / form.lanes);
-  if (run && !(phases & kPhaseWalk) && plan.schedule == SEGTACO_EB_SR) {
+  if (run && !(phases & kPhaseWalk) && plan.schedule == SEGTACO_EB_SR && form.own) {
     SegArgs g;
-    if (const int32_t sv =
-            seg_plan(b_dtype, a, ceil_div(L.ntiles, tiles_per_block) * a.panels, &g)) {
+    if (const int32_t sv = seg_plan(b_dtype, a, seg_walk_blocks(form, L.ntiles), &g)) {
       SEGTACO_HIP(mark(1));
       SEGTACO_HIP(launch_seg(b_dtype, sv, g, stream));
       SEGTACO_HIP(mark(2));
@@ -748,6 +763,34 @@ int32_t spmm_impl(const segtaco_csr_t *A, const void *B, int32_t b_dtype,
   SEGTACO_HIP(mark(2));
   SEGTACO_HIP(launch_fixup(V, a, stream));
   SEGTACO_HIP(mark(3));
+  return SEGTACO_OK;
+}
+
+int32_t spmm_form_impl(const segtaco_csr_t *A, const void *B, int32_t b_dtype, int64_t ldb,
+                       int32_t N, const float *C, int64_t ldc, const segtaco_plan_t *plan_in,
+                       bool batch, int32_t *out) {
+  if (!A || !plan_in || !out)
+    return set_error(SEGTACO_ERR_INVALID, "segtaco_spmm_form: null argument");
+  if (A->M < 1 || A->nnz < 1 || N < 1)
+    return set_error(SEGTACO_ERR_INVALID, "segtaco_spmm_form: empty product");
+  segtaco_plan_t plan = *plan_in;
+  SEGTACO_RET(resolve(A, N, b_dtype, ldb, ldc, B, C, &plan));
+  const ExecForm f = exec_form(plan, A->M, A->nnz, N, b_dtype,
+                               widest_vec(b_dtype, N, ldb, ldc, B, C));
+  out[0] = f.vec;
+  out[1] = f.lanes;
+  out[2] = out[3] = 0;
+  if (plan.schedule == SEGTACO_EB_SR && f.own && !batch) {
+    KArgs a{};
+    a.M = A->M;
+    a.N = N;
+    a.nnz = A->nnz;
+    a.tile = plan.tile;
+    a.ntiles = (int32_t)ceil_div(A->nnz, plan.tile);
+    SegArgs g;
+    out[2] = seg_plan(b_dtype, a, seg_walk_blocks(f, a.ntiles), &g);
+    out[3] = out[2] ? g.tpr : 0;
+  }
   return SEGTACO_OK;
 }
 
@@ -809,6 +852,12 @@ int32_t segtaco_spmm_workspace_layout(const segtaco_csr_t *A, int32_t N,
 int32_t segtaco_cs_workspace_layout(const segtaco_csr_t *A, int32_t N,
                                     const segtaco_plan_t *plan, int64_t *out) {
   return cs_workspace_layout_impl(A, N, plan, out);
+}
+
+int32_t segtaco_spmm_form(const segtaco_csr_t *A, const void *B, int32_t b_dtype,
+                          int64_t ldb, int32_t N, const float *C, int64_t ldc,
+                          const segtaco_plan_t *plan, int32_t batch, int32_t *out) {
+  return spmm_form_impl(A, B, b_dtype, ldb, N, C, ldc, plan, batch != 0, out);
 }
 
 int32_t segtaco_tile_rows(const int32_t *pos, int32_t M, int32_t tile, int32_t ntiles,

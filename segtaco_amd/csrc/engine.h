@@ -89,13 +89,25 @@ int32_t plan_resolve_ptrs_impl(const segtaco_csr_t *A, int32_t N, int32_t b_dtyp
                                int64_t ldb, int64_t ldc, const void *B, const void *C,
                                segtaco_plan_t *plan);
 
-// The vector width and lanes per B row a resolved plan runs with, in a call
-// of its own (alone) or in a batch.
+// Widest per-lane vector (in elements) that N, the leading dimensions and the
+// base pointers allow.
+int32_t widest_vec(int32_t dt, int32_t N, int64_t ldb, int64_t ldc, const void *B,
+                   const void *C);
+
+// The vector width and lanes per B row a resolved plan runs with; widest: as
+// widest_vec gives for the operands.
 struct ExecForm {
   int32_t vec, lanes, lq, panels;
+  // the plan leaves the form open: its vec is the widest the operands allow and
+  // its lanes are those a row spreads over
+  bool own;
 };
 ExecForm exec_form(const segtaco_plan_t &p, int32_t M, int32_t nnz, int32_t N,
-                   int32_t b_dtype);
+                   int32_t b_dtype, int32_t widest);
+// segtaco_spmm_form.
+int32_t spmm_form_impl(const segtaco_csr_t *A, const void *B, int32_t b_dtype, int64_t ldb,
+                       int32_t N, const float *C, int64_t ldc, const segtaco_plan_t *plan,
+                       bool batch, int32_t *out);
 
 // Default element-balanced tile of a product with nnz entries: `tile`,
 // halved (not below 8) while the product would have fewer than two

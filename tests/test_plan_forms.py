@@ -33,3 +33,46 @@ def test_eb_cs_sizing_of_unusual_plans(call, vec, lanes):
         A = S.csr_desc(1000, 1000, 5000, 0x1000, 0x2000, 0x3000, S.DT_F32)
         full = S.make_plan("eb_cs", vec=vec, col_lanes=8, group=64, tile=64, comp_threshold=0)
         assert r.stdout.strip() == str(S.cs_workspace_layout(A, 64, full))
+
+
+def _form(N, dtype, sched="eb_sr", M=60000, nnz=1_000_000, ldb=None, B=0, batch=False, **kw):
+    A = S.csr_desc(M, M, nnz, 0x1000, 0x2000, 0x3000, S.DTYPES[dtype])
+    return S.spmm_form(A, N, S.DTYPES[dtype], S.make_plan(sched, **kw), ldb, ldb, B, 0, batch)
+
+
+# A form that the plan names is the one that runs; each row once gave another's.
+@pytest.mark.parametrize("sched,dtype,N,kw", [
+    ("eb_sr", "f32", 64, dict(vec=1)), ("eb_sr", "f32", 64, dict(vec=2)),
+    ("eb_sr", "bf16", 64, dict(vec=4)), ("eb_sr", "f32", 4, dict(vec=1)),
+    ("eb_sr", "f32", 128, dict(vec=4, col_lanes=8)), ("rb_sr", "f32", 256, dict(vec=1)),
+    ("rb_pr", "f32", 128, dict(vec=1)), ("rb_pr", "bf16", 128, dict(vec=2, group=8)),
+    ("eb_pr", "f32", 128, dict(vec=1)), ("eb_pr", "bf16", 128, dict(vec=4))],
+    ids=lambda v: str(v) if not isinstance(v, dict) else "-".join(f"{k}{x}" for k, x in v.items()))
+@pytest.mark.parametrize("batch", [False, True])
+def test_named_slices_are_kept(sched, dtype, N, kw, batch):
+    f = _form(N, dtype, sched, tile=128 if sched[:2] == "eb" else 0, batch=batch, **kw)
+    A = S.csr_desc(60000, 60000, 1_000_000, 0x1000, 0x2000, 0x3000, S.DTYPES[dtype])
+    p = S.plan_resolve(A, N, S.DTYPES[dtype], S.make_plan(sched, **kw))
+    assert f == dict(vec=kw["vec"], lanes=p.col_lanes, seg_vec=0, seg_tiles=0)
+
+
+# The presets of one schedule that differ in their columns per lane run apart.
+@pytest.mark.parametrize("N", [32, 64])
+def test_column_presets_differ(N):
+    forms = [_form(N, "f32", "eb_sr", tile=256, vec=c) for c in (1, 2, 4)]
+    assert len({(f["vec"], f["lanes"], f["seg_vec"]) for f in forms}) >= 2
+    assert [f["vec"] for f in forms[:2]] == [1, 2]
+
+
+# Open plans, and plans resolved from them, keep the widths chosen for the call.
+def test_open_plans_choose():
+    assert _form(77, "fp16", tile=128)["vec"] == 4
+    assert _form(77, "f32", "rb_pr")["vec"] > 1
+    assert _form(128, "f32", ldb=129, tile=128)["vec"] == 4
+    assert _form(128, "f32", B=0x1004, tile=128)["vec"] == 4
+    assert _form(4, "f32")["seg_vec"] == 4
+    A = S.csr_desc(60000, 60000, 1_000_000, 0x1000, 0x2000, 0x3000, S.DT_F32)
+    for N in (4, 16, 64, 77, 128):
+        p = S.plan_resolve(A, N, S.DT_F32, S.make_plan("eb_sr"))
+        assert S.spmm_form(A, N, S.DT_F32, p) == S.spmm_form(A, N, S.DT_F32,
+                                                             S.make_plan("eb_sr"))
