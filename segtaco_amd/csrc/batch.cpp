@@ -101,7 +101,7 @@ void fill_batch_desc(const segtaco_csr_t &A, const void *B, int64_t ldb,
   a.C = C;
   a.ldc = ldc;
   const ExecForm form =
-      exec_form(plan, A.M, A.nnz, N, b_dtype, widest_vec(b_dtype, N, ldb, ldc, B, C));
+      exec_form(plan, A.M, A.nnz, N, b_dtype, widest_vec(b_dtype, N, ldb, ldc, B, C), true);
   a.lq = form.lq;
   a.lg = ilog2(plan.group);
   a.tile = plan.tile;

@@ -355,8 +355,19 @@ int32_t cs_vec(const segtaco_plan_t &p, int32_t N, int32_t b_dtype) {
 // N = 32 FP32 125, two elements 112). So do its products in a batch (12 power-law
 // products of 2000 to 20000 rows: BF16 N <= 64 286 / 119, FP32 N <= 64 164 / 118;
 // 24 of up to 200000 rows, FP32 N <= 128 2440 / 2320).
+//
+// Narrow slices mean fewer tiles per workgroup, which short tiles do not repay.
+// A batch pays for every unit it takes (an atomic, a search, the staging), so
+// where narrow slices would leave a unit less than 1024 entries it runs slices of
+// 4 columns, and of 8 where those would leave it 256 (power-law, one product, us per launch, widest /
+// narrow: 400 K entries FP32 N = 32 tile 16 47 / 77, tile 64 50 / 48, tile 128 68 / 54;
+// 2.4 M BF16 N = 16 tile 32 94 / 114, tile 64 148 / 94; N = 128 tile 16 154 / 323). A
+// call of its own launches its workgroups directly and loses only at the tiles
+// that small products resolve to (uniform rows, 1 M entries, slices of 1 / 2 / 4
+// columns: FP32 tile 8 N = 16 50 / 54 / 36, N = 64 - / 78 / 73; tile 16 N = 16 36 / 39 /
+// 32, N = 32 47 / 40 / 42; tile 32 N = 16 32 / 36 / 28; power-law tile 32 45 / 52 / 44).
 ExecForm exec_form(const segtaco_plan_t &p, int32_t M, int32_t nnz, int32_t N,
-                   int32_t b_dtype, int32_t widest) {
+                   int32_t b_dtype, int32_t widest, bool batch) {
   ExecForm f{p.vec, p.col_lanes, 0, 1, false};
   const int32_t w = widest_any(b_dtype, N);
   const bool open_vec = p.vec >= widest;
@@ -376,6 +387,14 @@ ExecForm exec_form(const segtaco_plan_t &p, int32_t M, int32_t nnz, int32_t N,
       if (f.own) {
         f.vec = N > 16 && nnz > 1200000 ? 2 : 1;
         while (f.vec < w && f.vec < 4 && 32 * f.vec < N) f.vec <<= 1;
+        int32_t least = 1;
+        if (batch) {
+          if (4 * natural_lanes(N, f.vec) > p.tile) least = 4;
+          if (natural_lanes(N, 4) >= p.tile) least = 8;
+        } else if (p.tile <= 16) {
+          least = p.tile > 8 && N > 16 && N <= 32 ? 2 : 4;
+        }
+        f.vec = std::max(f.vec, std::min(least, p.vec));
         f.lanes = natural_lanes(N, f.vec);
       }
       items = ceil_div(nnz, p.tile);
@@ -600,7 +619,8 @@ int32_t spmm_impl(const segtaco_csr_t *A, const void *B, int32_t b_dtype,
   a.C = C;
   a.ldc = ldc;
   const ExecForm form = exec_form(plan, A->M, A->nnz, N, b_dtype,
-                                  widest_vec(b_dtype, N, ldb, ldc, B, C));
+                                  widest_vec(b_dtype, N, ldb, ldc, B, C),
+                                  (phases & kPhaseWalk) != 0);
   const int32_t V = form.vec;
   a.lq = form.lq;
   // rb_sr's rows per group only order the launch: one row per group keeps
@@ -776,7 +796,7 @@ int32_t spmm_form_impl(const segtaco_csr_t *A, const void *B, int32_t b_dtype, i
   segtaco_plan_t plan = *plan_in;
   SEGTACO_RET(resolve(A, N, b_dtype, ldb, ldc, B, C, &plan));
   const ExecForm f = exec_form(plan, A->M, A->nnz, N, b_dtype,
-                               widest_vec(b_dtype, N, ldb, ldc, B, C));
+                               widest_vec(b_dtype, N, ldb, ldc, B, C), batch);
   out[0] = f.vec;
   out[1] = f.lanes;
   out[2] = out[3] = 0;

@@ -66,7 +66,7 @@ int32_t device_cus();
 constexpr int32_t kPhasePrepare = 1;
 constexpr int32_t kPhaseRun = 2;
 constexpr int32_t kPhaseAll = kPhasePrepare | kPhaseRun;
-// Beside kPhaseAll: eb_sr as a batch runs it, never in the segment form.
+// Beside kPhaseAll: eb_sr in the form that a batch runs.
 constexpr int32_t kPhaseWalk = 4;
 
 // The device API's implementation (engine.cpp). ev: 4 optional events
@@ -94,8 +94,8 @@ int32_t plan_resolve_ptrs_impl(const segtaco_csr_t *A, int32_t N, int32_t b_dtyp
 int32_t widest_vec(int32_t dt, int32_t N, int64_t ldb, int64_t ldc, const void *B,
                    const void *C);
 
-// The vector width and lanes per B row a resolved plan runs with; widest: as
-// widest_vec gives for the operands.
+// The vector width and lanes per B row a resolved plan runs with, in a call of
+// its own or in a batch; widest: as widest_vec gives for the operands.
 struct ExecForm {
   int32_t vec, lanes, lq, panels;
   // the plan leaves the form open: its vec is the widest the operands allow and
@@ -103,7 +103,7 @@ struct ExecForm {
   bool own;
 };
 ExecForm exec_form(const segtaco_plan_t &p, int32_t M, int32_t nnz, int32_t N,
-                   int32_t b_dtype, int32_t widest);
+                   int32_t b_dtype, int32_t widest, bool batch);
 // segtaco_spmm_form.
 int32_t spmm_form_impl(const segtaco_csr_t *A, const void *B, int32_t b_dtype, int64_t ldb,
                        int32_t N, const float *C, int64_t ldc, const segtaco_plan_t *plan,

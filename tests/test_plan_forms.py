@@ -76,3 +76,19 @@ def test_open_plans_choose():
         p = S.plan_resolve(A, N, S.DT_F32, S.make_plan("eb_sr"))
         assert S.spmm_form(A, N, S.DT_F32, p) == S.spmm_form(A, N, S.DT_F32,
                                                              S.make_plan("eb_sr"))
+
+
+# Short tiles keep wide slices: a batch's unit holds 1024 entries where slices of
+# four columns allow it, and a call's tiles of up to 16 entries are not spread thin.
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("N", [4, 8, 16, 24, 32, 64, 128, 256])
+@pytest.mark.parametrize("tile", [8, 16, 32, 64, 128])
+def test_short_tiles_keep_wide_slices(N, tile, dtype):
+    f = _form(N, dtype, tile=tile, batch=True)
+    widest = min(4 if dtype == "f32" else 8, N)
+    assert tile * 256 // f["lanes"] >= 1024 or f["vec"] >= min(4, widest)
+    assert tile > f["lanes"] or f["vec"] == widest
+    if tile <= 16 and N > 8:
+        assert _form(N, dtype, tile=tile, M=1_000_000, nnz=1_500_000)["vec"] >= 2
+    if tile == 128:  # the narrow forms
+        assert f["vec"] == max(1, min(4, N // 32))
