@@ -414,8 +414,12 @@ int32_t seg_plan(int32_t dt, const KArgs &a, int64_t walk_blocks, SegArgs *g) {
   // and BF16, us per call, walk / segments:
   //   up to 8 columns: segments at every size (above, and 262144^2 N = 8:
   //     144 / 95 and 129 / 95);
-  //   9 to 16: 60000^2 (1 M entries) 81 / 36 and 56 / 43; 200000^2 (2.4 M) 93 /
-  //     79 and 74 / 82; 262144^2 (4.2 M) 116 / 126: up to 24 M products;
+  //   9 to 16 (N = 16, tile 128): 500 K entries 40 / 25 and 39 / 27, 960 K 43 /
+  //     35 and 40 / 46, 1.2 M 41 / 42 and 38 / 54: up to 2^20 entries in FP32, 2^19
+  //     in 16 bits, whose slices of 8 gather more columns than N has. Short
+  //     tiles cut more pieces, and uniform rows, which the walk takes best, lose
+  //     (FP32, tile 16, power-law and uniform: 500 K 47 / 35 and 22 / 26, 1 M 50 / 46
+  //     and 32 / 40; BF16 1 M 65 / 62 and 33 / 50): up to 2^19 entries;
   //   17 to 64: small products (1000^2, 15.6 K entries, N = 64: 36 / 22 at
   //     tile 128, 21 / 13 at tile 8), and where the walk leaves half of the
   //     chip without a workgroup: 8000^2 N = 64 (63 workgroups) 43 / 28, but
@@ -424,8 +428,9 @@ int32_t seg_plan(int32_t dt, const KArgs &a, int64_t walk_blocks, SegArgs *g) {
   // rows per wave, so mostly empty matrices keep the row-parallel partition.
   if (a.tile > kSegMaxRange || a.N > 64 || (int64_t)a.M > 2 * (int64_t)a.nnz) return 0;
   const int64_t products = (int64_t)a.nnz * a.N;
+  const int32_t most = dt == 0 && a.tile >= 64 ? 1 << 20 : 1 << 19;  // entries, N 9 to 16
   const bool take = a.N <= 8    ? true
-                    : a.N <= 16 ? products <= 24000000
+                    : a.N <= 16 ? a.nnz <= most
                                 : products <= 2000000 ||
                                       (products <= 12000000 && walk_blocks < 128);
   if (!take) return 0;

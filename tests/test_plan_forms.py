@@ -92,3 +92,20 @@ def test_short_tiles_keep_wide_slices(N, tile, dtype):
         assert _form(N, dtype, tile=tile, M=1_000_000, nnz=1_500_000)["vec"] >= 2
     if tile == 128:  # the narrow forms
         assert f["vec"] == max(1, min(4, N // 32))
+
+
+# The segment form takes narrow products of any size, those of 9 to 16 columns up
+# to the size from which the walk is faster, and never a plan that names its slices.
+@pytest.mark.parametrize("dtype,tile,N,nnz,seg", [
+    ("f32", 128, 8, 4_000_000, True), ("bf16", 16, 8, 4_000_000, True),
+    ("f32", 128, 16, 1 << 20, True), ("f32", 128, 16, (1 << 20) + 1, False),
+    ("f32", 64, 9, 1 << 20, True), ("f32", 32, 9, (1 << 19) + 1, False),
+    ("f32", 16, 12, 1 << 19, True), ("f32", 16, 12, 1_000_000, False),
+    ("bf16", 128, 16, 1 << 19, True), ("bf16", 128, 12, 1_000_000, False),
+    ("fp16", 16, 9, 2_000_000, False), ("f32", 128, 17, 1 << 20, False)])
+def test_segment_form_by_size(dtype, tile, N, nnz, seg):
+    assert (_form(N, dtype, nnz=nnz, tile=tile)["seg_vec"] > 0) == seg
+    assert _form(N, dtype, nnz=nnz, tile=tile, batch=True)["seg_vec"] == 0
+    assert _form(N, dtype, nnz=nnz, M=2 * nnz + 1, tile=tile)["seg_vec"] == 0
+    if N % 2 == 0:
+        assert _form(N, dtype, nnz=nnz, tile=tile, vec=1)["seg_vec"] == 0
