@@ -219,7 +219,10 @@ __device__ __forceinline__ void rb_sr_body(const KArgs &a, int32_t blk,
 // rb_pr over row block `blk`, column panel `panel`: R sets of 64/(P*Q) rows per
 // wave. A row of up to P entries is one step (row pointer, column, gather) of
 // three dependent loads, so a wave with several sets has them in flight
-// together.
+// together. The block's waves take its sets in turn: a wave sums the rest of its
+// longer rows one set after another, and adjacent rows are often alike (lengths
+// in rising order, 100000^2, us per call, a wave's sets adjacent / so: FP32 N = 3
+// 65 / 57, N = 8 69 / 63, BF16 N = 12 163 / 135; one set per wave 47, 44, 131).
 template <int DT, int V, bool kOff32, int R>
 __device__ __forceinline__ void rb_pr_walk(const KArgs &a, int32_t blk,
                                            int32_t panel) {
@@ -227,7 +230,8 @@ __device__ __forceinline__ void rb_pr_walk(const KArgs &a, int32_t blk,
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lq = a.lq, lg = a.lg;
   const int lr = 6 - lq - lg;  // log2(rows per set)
-  const int64_t row0 = ((int64_t)blk * kWavesPerBlock + wave) * R << lr;
+  const int64_t row0 = ((int64_t)blk * kWavesPerBlock * R + wave) << lr;
+  const int64_t set = (int64_t)kWavesPerBlock << lr;  // rows to the wave's next set
   if (row0 >= a.M) return;  // uniform over the wave
   const int32_t slot = (lane >> lq) & ((1 << lg) - 1);
   const int32_t P = 1 << lg;
@@ -240,7 +244,7 @@ __device__ __forceinline__ void rb_pr_walk(const KArgs &a, int32_t blk,
   bool comp[R];
 #pragma unroll
   for (int k = 0; k < R; ++k) {
-    const int64_t row = row0 + ((int64_t)k << lr) + (lane >> (lq + lg));
+    const int64_t row = row0 + k * set + (lane >> (lq + lg));
     const bool live = row < a.M && colok;
     const int32_t s = live ? a.pos[row] : 0;
     const int32_t len = live ? a.pos[row + 1] - s : 0;
@@ -292,7 +296,7 @@ __device__ __forceinline__ void rb_pr_walk(const KArgs &a, int32_t blk,
   for (int k = 0; k < R; ++k) butterfly<V>(acc[k], P << lq >> 1, 1 << lq);
 #pragma unroll
   for (int k = 0; k < R; ++k) {
-    const int64_t row = row0 + ((int64_t)k << lr) + (lane >> (lq + lg));
+    const int64_t row = row0 + k * set + (lane >> (lq + lg));
     if (row < a.M && colok && slot == 0) store_row<V>(a.C + row * a.ldc + col, acc[k]);
   }
 }
