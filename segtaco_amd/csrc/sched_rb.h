@@ -141,7 +141,10 @@ __device__ __forceinline__ void rb_sr_row(const KArgs &a, int32_t row, int32_t p
   store_row<V>(a.C + (int64_t)row * a.ldc + col, acc);
 }
 
-// The sum of the n > 0 entries p, p + 2^lg, ... of a slot of rb_pr.
+// The sum of the n > 0 entries p, p + 2^lg, ... of a slot of rb_pr. A batch loads
+// no entries that are not there: where B stays in the caches the loads themselves
+// are the time (banded, 33 entries per row, 8 slots, us per call, all four loads /
+// those needed: FP32 N = 4 21 / 16, N = 64 176 / 159, BF16 N = 1 18 / 14).
 template <int DT, int V, bool kOff32, bool kComp>
 __device__ __forceinline__ void rb_pr_sum(const KArgs &a, int32_t p, int32_t n, int lg,
                                           int32_t col, float (&acc)[V]) {
@@ -149,14 +152,24 @@ __device__ __forceinline__ void rb_pr_sum(const KArgs &a, int32_t p, int32_t n, 
   constexpr int U = 4;
   float cmp[V], v[U];
   zero_vec(cmp);
-  const int32_t last = p + ((n - 1) << lg);
   int32_t c[U];
   auto entries = [&](int32_t b) {
+    if (b + U <= n) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int32_t i = b + u < n ? p + ((b + u) << lg) : last;
-      c[u] = a.crd[i];
-      v[u] = load_val<DT>(a.vals, i);
+      for (int u = 0; u < U; ++u) {
+        const int32_t i = p + ((b + u) << lg);
+        c[u] = a.crd[i];
+        v[u] = load_val<DT>(a.vals, i);
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (b + u < n) {
+          const int32_t i = p + ((b + u) << lg);
+          c[u] = a.crd[i];
+          v[u] = load_val<DT>(a.vals, i);
+        }
+      }
     }
   };
   entries(0);
@@ -175,7 +188,8 @@ __device__ __forceinline__ void rb_pr_sum(const KArgs &a, int32_t p, int32_t n, 
   }
   if (b < n) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) x[u] = load_row_raw<DT, V, kOff32>(a.B, c[u], a.ldb, col);
+    for (int u = 0; u < U; ++u)
+      if (b + u < n) x[u] = load_row_raw<DT, V, kOff32>(a.B, c[u], a.ldb, col);
 #pragma unroll
     for (int u = 0; u < U; ++u) rb_add_if<DT, V, kComp>(b + u < n, x[u], v[u], acc, cmp);
   }
@@ -257,8 +271,12 @@ __device__ __forceinline__ void rb_pr_walk(const KArgs &a, int32_t blk,
   for (int k = 0; k < R; ++k) zero_vec(acc[k]);
   if (R > 1 || __ballot(n[0] > 1) == 0) {
     // each slot's first entry, all sets' loads in flight together (a slot
-    // without one reads entry 0)
-    if (a.nnz > 0) {
+    // without one reads entry 0; a wave of empty rows loads nothing: two rows in
+    // three empty, BF16 N = 128 110 / 90 us per call)
+    bool some = false;
+#pragma unroll
+    for (int k = 0; k < R; ++k) some = some || n[k] > 0;
+    if (__ballot(some) != 0) {
       int32_t c[R];
       float v[R];
       typename RawT<DT, V>::type x[R];
