@@ -16,8 +16,7 @@
 //
 // Both walk in batches whose gathers are in flight together. A batch's
 // columns and values are loaded during the batch before it, so a batch costs
-// one memory latency, not two; every load is unconditional, so a row's last,
-// partial batch costs one latency too, and no wait covers more than its batch.
+// one memory latency, not two, and a row's last, partial batch one too.
 //
 // Neither schedule needs C cleared first: every row (empty ones included) is
 // written exactly once.
@@ -93,9 +92,13 @@ struct RbEntries {
 };
 
 // The sum of entries p .. e - 1 (p < e) for this lane's V columns. Whole
-// batches run without a predicate on their entries; the last, partial one
-// gathers its first entry's row in the place of missing ones.
-// kRun: entries up to e + 2 * U - 2 exist.
+// batches run without a predicate on their entries. The wave's last batch loads
+// no entries after it and a partial one gathers only rows that are there (short
+// rows: two in three empty, the others of 8, FP32, us per call without / with these:
+// N = 32 24 / 21, N = 50 69 / 54; banded, 33 entries per row: N = 64 88 / 78, N = 128 172 /
+// 151; uniform 20 entries N = 32 31 / 31); a compensated row is long, and the test
+// in its loop would cost more than the loads (lengths in rising order, BF16
+// N = 3 173 / 224). kRun: entries up to e + 2 * U - 2 exist.
 template <int DT, int V, bool kOff32, int U, bool kRun, bool kComp>
 __device__ __forceinline__ void rb_sr_sum(const KArgs &a, int32_t p, int32_t e, int32_t col,
                                           float (&acc)[V]) {
@@ -109,18 +112,26 @@ __device__ __forceinline__ void rb_sr_sum(const KArgs &a, int32_t p, int32_t e, 
 #pragma unroll
     for (int u = 0; u < U; ++u)
       x[u] = load_row_raw<DT, V, kOff32>(a.B, m.c[u], a.ldb, col);
+    if (!kComp && __ballot(e - p > U) == 0) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) rb_add<DT, V, kComp>(x[u], m.val(a, u), acc, cmp);
+      p = e;
+      break;
+    }
     const RbEntries<DT, kRun, U> w = m;
     m.load(a, kRun ? p + U : min(p + U, e - 1), e - 1);
 #pragma unroll
     for (int u = 0; u < U; ++u) rb_add<DT, V, kComp>(x[u], w.val(a, u), acc, cmp);
   }
   if (p < e) {
+    R y[U] = {};
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      x[u] = load_row_raw<DT, V, kOff32>(a.B, u < e - p ? m.c[u] : m.c[0], a.ldb, col);
+      if (kComp || u < e - p)
+        y[u] = load_row_raw<DT, V, kOff32>(a.B, u < e - p ? m.c[u] : m.c[0], a.ldb, col);
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      rb_add_if<DT, V, kComp>(u < e - p, x[u], m.val(a, u), acc, cmp);
+      rb_add_if<DT, V, kComp>(u < e - p, y[u], m.val(a, u), acc, cmp);
   }
   if constexpr (kComp) {
 #pragma unroll
