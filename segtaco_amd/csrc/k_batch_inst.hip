@@ -29,7 +29,7 @@ __device__ __forceinline__ void run_body(int32_t sched, const KArgs &a,
     return;
   }
   switch (sched) {
-    case SEGTACO_RB_SR: rb_sr_body<DT, V>(a, blk, panel); break;
+    case SEGTACO_RB_SR: rb_sr_body<DT, V, true>(a, blk, panel); break;
     case SEGTACO_RB_PR: rb_pr_body<DT, V>(a, blk, panel); break;
     case SEGTACO_EB_SR: eb_sr_body<DT, V>(a, blk, panel, smem); break;
     default:

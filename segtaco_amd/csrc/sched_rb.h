@@ -98,8 +98,10 @@ struct RbEntries {
 // N = 32 24 / 21, N = 50 69 / 54; banded, 33 entries per row: N = 64 88 / 78, N = 128 172 /
 // 151; uniform 20 entries N = 32 31 / 31); a compensated row is long, and the test
 // in its loop would cost more than the loads (lengths in rising order, BF16
-// N = 3 173 / 224). kRun: entries up to e + 2 * U - 2 exist.
-template <int DT, int V, bool kOff32, int U, bool kRun, bool kComp>
+// N = 3 173 / 224). kLean: without these, for the batched kernel, where their
+// registers would spill (BF16 88 bytes).
+// kRun: entries up to e + 2 * U - 2 exist.
+template <int DT, int V, bool kOff32, int U, bool kRun, bool kComp, bool kLean>
 __device__ __forceinline__ void rb_sr_sum(const KArgs &a, int32_t p, int32_t e, int32_t col,
                                           float (&acc)[V]) {
   using R = typename RawT<DT, V>::type;
@@ -112,7 +114,7 @@ __device__ __forceinline__ void rb_sr_sum(const KArgs &a, int32_t p, int32_t e, 
 #pragma unroll
     for (int u = 0; u < U; ++u)
       x[u] = load_row_raw<DT, V, kOff32>(a.B, m.c[u], a.ldb, col);
-    if (!kComp && __ballot(e - p > U) == 0) {
+    if (!kComp && !kLean && __ballot(e - p > U) == 0) {
 #pragma unroll
       for (int u = 0; u < U; ++u) rb_add<DT, V, kComp>(x[u], m.val(a, u), acc, cmp);
       p = e;
@@ -127,7 +129,7 @@ __device__ __forceinline__ void rb_sr_sum(const KArgs &a, int32_t p, int32_t e, 
     R y[U] = {};
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (kComp || u < e - p)
+      if (kComp || kLean || u < e - p)
         y[u] = load_row_raw<DT, V, kOff32>(a.B, u < e - p ? m.c[u] : m.c[0], a.ldb, col);
 #pragma unroll
     for (int u = 0; u < U; ++u)
@@ -140,15 +142,15 @@ __device__ __forceinline__ void rb_sr_sum(const KArgs &a, int32_t p, int32_t e, 
 }
 
 // One output row of rb_sr (entries p .. e - 1) for this lane's V columns.
-template <int DT, int V, bool kOff32, int U, bool kRun>
+template <int DT, int V, bool kOff32, int U, bool kRun, bool kLean>
 __device__ __forceinline__ void rb_sr_row(const KArgs &a, int32_t row, int32_t p, int32_t e,
                                           int32_t col) {
   float acc[V];
   zero_vec(acc);
   if (e - p > a.comp_threshold)
-    rb_sr_sum<DT, V, kOff32, U, kRun, true>(a, p, e, col, acc);
+    rb_sr_sum<DT, V, kOff32, U, kRun, true, kLean>(a, p, e, col, acc);
   else if (p < e)
-    rb_sr_sum<DT, V, kOff32, U, kRun, false>(a, p, e, col, acc);
+    rb_sr_sum<DT, V, kOff32, U, kRun, false, kLean>(a, p, e, col, acc);
   store_row<V>(a.C + (int64_t)row * a.ldc + col, acc);
 }
 
@@ -211,9 +213,10 @@ __device__ __forceinline__ void rb_pr_sum(const KArgs &a, int32_t p, int32_t n, 
 }
 
 // rb_sr over row block `blk`, column panel `panel`: lane group gi owns row gi.
-template <int DT, int V, int U, bool kOff32>
+template <int DT, int V, bool kLean, bool kOff32>
 __device__ __forceinline__ void rb_sr_walk(const KArgs &a, int32_t blk,
                                            int32_t panel) {
+  constexpr int U = 8;  // entries per batch
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int lq = a.lq;
@@ -227,18 +230,18 @@ __device__ __forceinline__ void rb_sr_walk(const KArgs &a, int32_t blk,
   const bool run = __ballot(live && a.nnz - e < 2 * U) == 0;
   if (!live) return;
   if (run)
-    rb_sr_row<DT, V, kOff32, U, true>(a, (int32_t)row, p, e, col);
+    rb_sr_row<DT, V, kOff32, U, true, kLean>(a, (int32_t)row, p, e, col);
   else
-    rb_sr_row<DT, V, kOff32, U, false>(a, (int32_t)row, p, e, col);
+    rb_sr_row<DT, V, kOff32, U, false, kLean>(a, (int32_t)row, p, e, col);
 }
 
-template <int DT, int V, int U = 8>
+template <int DT, int V, bool kLean = false>
 __device__ __forceinline__ void rb_sr_body(const KArgs &a, int32_t blk,
                                            int32_t panel) {
   if (a.b_off32)
-    rb_sr_walk<DT, V, U, true>(a, blk, panel);
+    rb_sr_walk<DT, V, kLean, true>(a, blk, panel);
   else
-    rb_sr_walk<DT, V, U, false>(a, blk, panel);
+    rb_sr_walk<DT, V, kLean, false>(a, blk, panel);
 }
 
 // rb_pr over row block `blk`, column panel `panel`: R sets of 64/(P*Q) rows per
