@@ -359,9 +359,11 @@ int32_t cs_vec(const segtaco_plan_t &p, int32_t N, int32_t b_dtype) {
 // Narrow slices mean fewer tiles per workgroup, which short tiles do not repay.
 // A batch pays for every unit it takes (an atomic, a search, the staging), so
 // where narrow slices would leave a unit less than 1024 entries it runs slices of
-// 4 columns, and of 8 where those would leave it 256 (power-law, one product, us per launch, widest /
-// narrow: 400 K entries FP32 N = 32 tile 16 47 / 77, tile 64 50 / 48, tile 128 68 / 54;
-// 2.4 M BF16 N = 16 tile 32 94 / 114, tile 64 148 / 94; N = 128 tile 16 154 / 323). A
+// 2 or 4 columns (power-law, 16 products of 1 and 2.4 M entries, us per launch,
+// narrow / so: FP32 N = 16 tile 32 873 / 647, N = 64 tile 64 1173 / 1089, BF16 N = 32
+// tile 32 1148 / 846; N = 32 tile 64, slices of 1 / 2 / 4 BF16 834 / 691 / 851), never of
+// 8, since one product of those would take its whole batch to the kernel with
+// every schedule (alone, 2.4 M entries, BF16 N = 64 tile 8: 214 / 316 with 8 / 4). A
 // call of its own launches its workgroups directly and loses only at the tiles
 // that small products resolve to (uniform rows, 1 M entries, slices of 1 / 2 / 4
 // columns: FP32 tile 8 N = 16 50 / 54 / 36, N = 64 - / 78 / 73; tile 16 N = 16 36 / 39 /
@@ -389,8 +391,8 @@ ExecForm exec_form(const segtaco_plan_t &p, int32_t M, int32_t nnz, int32_t N,
         while (f.vec < w && f.vec < 4 && 32 * f.vec < N) f.vec <<= 1;
         int32_t least = 1;
         if (batch) {
-          if (4 * natural_lanes(N, f.vec) > p.tile) least = 4;
-          if (natural_lanes(N, 4) >= p.tile) least = 8;
+          if (4 * natural_lanes(N, f.vec) > p.tile)
+            least = N > 16 && 4 * natural_lanes(N, 2) <= p.tile ? 2 : 4;
         } else if (p.tile <= 16) {
           least = p.tile > 8 && N > 16 && N <= 32 ? 2 : 4;
         }

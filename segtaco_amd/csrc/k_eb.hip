@@ -5,7 +5,7 @@
 
 namespace segtaco {
 
-size_t eb_sr_lds_bytes(const KArgs &a) { return eb_sr_lds_bytes_lq(a.lq); }
+size_t eb_sr_lds_bytes(const KArgs &a) { return eb_sr_lds_bytes_lq(a.lq, a.tile); }
 size_t eb_pr_lds_bytes(const KArgs &) { return eb_pr_lds_bytes_fixed(); }
 
 template <int V>

@@ -62,14 +62,18 @@ constexpr int kSrBatch = 4;
 constexpr int32_t kPrChunk = 128;
 constexpr int kPrPasses = 8;       // eb_pr passes whose gathers are in flight
 
-// eb_sr chunk: the LDS per block stays under 64 KiB for every lane count.
-__host__ __device__ inline int32_t eb_sr_chunk(int32_t lq) {
+// eb_sr chunk: the LDS per block stays under 64 KiB for every lane count, and a
+// short tile takes no more than its entries, since the LDS of a batch's largest
+// product decides how many workgroups all of them have (32 products, one of
+// them 4 lanes and tile 16, BF16: 4.3 ms per launch with 64-entry chunks, 3.5 so).
+__host__ __device__ inline int32_t eb_sr_chunk(int32_t lq, int32_t tile) {
   const int32_t c = 16 << lq;
-  return c < kSrChunkMax ? c : kSrChunkMax;
+  const int32_t whole = tile < kSrChunkMax ? (tile + 15) & ~15 : kSrChunkMax;
+  return c < whole ? c : whole;
 }
 
-__host__ __device__ inline size_t eb_sr_lds_bytes_lq(int32_t lq) {
-  const int32_t ch = eb_sr_chunk(lq);
+__host__ __device__ inline size_t eb_sr_lds_bytes_lq(int32_t lq, int32_t tile) {
+  const int32_t ch = eb_sr_chunk(lq, tile);
   const size_t groups = (size_t)kWavesPerBlock << (6 - lq);
   return groups * (size_t)(3 * ch + kPosSlack) * sizeof(int32_t);
 }
@@ -100,7 +104,7 @@ __device__ __forceinline__ void zero_empty_rows(const KArgs &a, int32_t r0,
 }
 
 // eb_sr over tile block `blk` (kWavesPerBlock * 64/Q tiles, one per lane
-// group), column panel `panel`; smem holds eb_sr_lds_bytes_lq(lq) bytes.
+// group), column panel `panel`; smem holds eb_sr_lds_bytes_lq(lq, tile) bytes.
 // kWide: some tile of the wave spans more rows than the chunk's LDS window of
 // the row pointer holds, so row lookups past the window read pos from memory.
 // Otherwise every lookup is an LDS read: a lookup that may go to either
@@ -116,7 +120,7 @@ __device__ __forceinline__ void eb_sr_walk(const KArgs &a, int32_t blk,
   const int32_t q = lane & (Q - 1);
   const int32_t gib = (wave << (6 - lq)) + (lane >> lq);  // group in block
   const int32_t t = blk * (kWavesPerBlock << (6 - lq)) + gib;
-  const int32_t CH = eb_sr_chunk(lq);
+  const int32_t CH = eb_sr_chunk(lq, a.tile);
   const int32_t PW = CH + kPosSlack;
   int32_t *s_crd = smem + gib * (3 * CH + kPosSlack);
   float *s_val = reinterpret_cast<float *>(s_crd + CH);
@@ -298,7 +302,7 @@ __device__ __forceinline__ void eb_sr_body(const KArgs &a, int32_t blk,
   const int wave = threadIdx.x >> 6;
   const int lq = a.lq;
   const int32_t t = blk * (kWavesPerBlock << (6 - lq)) + (wave << (6 - lq)) + (lane >> lq);
-  const int32_t PW = eb_sr_chunk(lq) + kPosSlack;
+  const int32_t PW = eb_sr_chunk(lq, a.tile) + kPosSlack;
   const bool wide = t < a.ntiles && a.tile_row[t + 1] - a.tile_row[t] > PW - 2;
   const bool any_wide = __ballot(wide) != 0;
   if (a.b_off32) {

@@ -85,9 +85,8 @@ def test_open_plans_choose():
 @pytest.mark.parametrize("tile", [8, 16, 32, 64, 128])
 def test_short_tiles_keep_wide_slices(N, tile, dtype):
     f = _form(N, dtype, tile=tile, batch=True)
-    widest = min(4 if dtype == "f32" else 8, N)
-    assert tile * 256 // f["lanes"] >= 1024 or f["vec"] >= min(4, widest)
-    assert tile > f["lanes"] or f["vec"] == widest
+    assert tile * 256 // f["lanes"] >= 1024 or f["vec"] == 4
+    assert f["vec"] <= 4  # eight columns would take the kernel with every schedule
     if tile <= 16 and N > 8:
         assert _form(N, dtype, tile=tile, M=1_000_000, nnz=1_500_000)["vec"] >= 2
     if tile == 128:  # the narrow forms
