@@ -4,7 +4,8 @@
  * No counterpart in the reference (one matrix per process, one kernel per
  * call, matrix_main.cpp:13-57). A batch fixes a set of device-resident
  * products C_i = A_i * B_i (each with its own shape, N_i and plan) and runs
- * them all with one persistent kernel whose workgroups pull work units from a
+ * them all with one persistent kernel (two where large eb_sr products meet other
+ * schedules) whose workgroups pull work units from a
  * shared counter, followed by one batched carry fix-up. Creating the batch
  * resolves every plan (the autotuner picks one from the row-length
  * statistics when the item's schedule is negative) and runs the per-matrix
@@ -51,7 +52,7 @@ int32_t segtaco_batch_run(segtaco_batch_t b, void *stream);
 int32_t segtaco_batch_capture(segtaco_batch_t b);
 /* Launches the captured graph on `stream` (asynchronous). */
 int32_t segtaco_batch_replay(segtaco_batch_t b, void *stream);
-/* Resolved plan of item i; number of work units of the persistent launch;
+/* Resolved plan of item i; number of work units of the persistent launches;
  * bytes of device workspace the batch holds. */
 int32_t segtaco_batch_plan(segtaco_batch_t b, int32_t i, segtaco_plan_t *out);
 int64_t segtaco_batch_units(segtaco_batch_t b);

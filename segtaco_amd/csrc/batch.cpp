@@ -3,10 +3,10 @@
 // Create: resolve each product's plan (tuned from its row-length statistics
 // when asked), lay out one device workspace for all element-balanced
 // products (partition, tile rows, carries), compute each product's work-unit
-// range, and run the row partitions once. Run: reset the unit counter, one
-// persistent launch over all units, one batched fix-up launch. The sequence
-// can be captured into a HIP graph (no memset nodes: the counter is cleared
-// by a kernel).
+// range, and run the row partitions once. Run: reset the unit counters, one
+// persistent launch over all units of the eb_sr products and one over the
+// others' (BatchPart), one batched fix-up launch. The sequence can be captured
+// into a HIP graph (no memset nodes: the counters are cleared by a kernel).
 #include <algorithm>
 #include <climits>
 #include <cstring>
@@ -25,20 +25,40 @@ int32_t plan_resolve_impl(const segtaco_csr_t *A, int32_t N, int32_t b_dtype,
 
 using namespace segtaco;
 
+// The products of one persistent launch. A mixed batch whose eb_sr products are
+// large runs them (part 0) in a kernel of their own, which holds more waves than
+// one that carries every schedule, and the others in part 1; else all share one.
+// prefix spans all products of the batch; those of the other part have no units.
+struct BatchPart {
+  std::vector<int64_t> prefix;
+  size_t lds = 0;
+  int32_t grid = 0;
+  BatchForm form = kBatchEbSr;  // the largest of its products'
+  int64_t units() const { return prefix.back(); }
+};
+constexpr int kParts = 2;
+// Entries of eb_sr products in slices of less than 4 columns from which a mixed
+// batch is split. The second launch costs 30 to 45 us, and the kernel of their own
+// saves 2 to 8 us per million entries: power-law products of 1 and 2.4 M entries and
+// one rb_sr product, us per launch in one part / two: FP32 N = 32, 4 products 241 /
+// 242, 16 763 / 690, 64 2881 / 2532; N = 64, 8 products 611 / 625, 32 2175 / 2133;
+// BF16 N = 64, 8 products 501 / 437, 32 1918 / 1512; slices of 4 gain nothing
+// (FP32 N = 128, 16 products 2137 / 2188).
+constexpr int64_t kSplitEntries = 1 << 24;
+constexpr size_t kCounterStride = 256;  // a cache line and more per counter
+
 struct segtaco_batch {
   int32_t n = 0, dt = 0;
   std::vector<BatchDesc> descs;
   std::vector<segtaco_plan_t> plans;
-  std::vector<int64_t> prefix, fix_prefix;
-  int64_t total_units = 0, total_fix = 0;
+  BatchPart parts[kParts];
+  std::vector<int64_t> fix_prefix;
+  int64_t total_fix = 0;
   BatchDesc *d_desc = nullptr;
-  int64_t *d_prefix = nullptr, *d_fix_prefix = nullptr;
-  unsigned long long *d_counter = nullptr;
+  int64_t *d_prefix = nullptr, *d_fix_prefix = nullptr;  // d_prefix: per part, n + 1
+  char *d_counter = nullptr;
   char *ws = nullptr;
   size_t ws_bytes = 0;
-  size_t lds = 0;
-  int32_t grid = 0;
-  BatchForm form = kBatchEbSr;  // the largest of its products'
   hipStream_t cap_stream = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -157,10 +177,13 @@ int32_t segtaco_batch_create(const segtaco_batch_item_t *items, int32_t n,
   b->dt = b_dtype;
   b->descs.resize(n);
   b->plans.resize(n);
-  b->prefix.resize(n + 1, 0);
+  for (auto &p : b->parts) p.prefix.resize(n + 1, 0);
   b->fix_prefix.resize(n + 1, 0);
   std::vector<size_t> ws_off(n, 0);
   std::vector<EbLayout> lay(n);
+  std::vector<int64_t> unit_count(n, 0);
+  std::vector<size_t> item_lds(n, 0);
+  int64_t narrow = 0;  // entries of eb_sr products in slices of less than 4 columns
   size_t ws_total = 0;
   int32_t st = SEGTACO_OK;
 
@@ -189,7 +212,6 @@ int32_t segtaco_batch_create(const segtaco_batch_item_t *items, int32_t n,
     std::memset(&D, 0, sizeof(D));
     if (A.M == 0 || it.N == 0) {
       b->plans[i] = plan;
-      b->prefix[i + 1] = b->prefix[i];
       b->fix_prefix[i + 1] = b->fix_prefix[i];
       continue;
     }
@@ -216,23 +238,32 @@ int32_t segtaco_batch_create(const segtaco_batch_item_t *items, int32_t n,
     size_t lds = 0;
     fill_batch_desc(A, it.B, it.ldb, it.C, it.ldc, it.N, b_dtype, plan, &D, &units,
                     &fix_units, &lds, &lay[i]);
-    if (lds > b->lds) b->lds = lds;
-    b->form = std::max(b->form, batch_form(D));
+    unit_count[i] = units;
+    item_lds[i] = lds;
+    if (batch_form(D) == kBatchEbSr && D.vec < 4) narrow += A.nnz;
     if (plan.schedule >= SEGTACO_EB_SR) {
       ws_off[i] = ws_total;
       ws_total += align_up(lay[i].total, 256);
     }
-    D.unit_begin = b->prefix[i];
     D.fix_begin = b->fix_prefix[i];
-    b->prefix[i + 1] = b->prefix[i] + units;
     b->fix_prefix[i + 1] = b->fix_prefix[i] + fix_units;
   }
   if (st != SEGTACO_OK) {
     release(b);
     return st;
   }
-  b->total_units = b->prefix[n];
   b->total_fix = b->fix_prefix[n];
+  const bool split = narrow >= kSplitEntries;
+  for (int32_t i = 0; i < n; ++i) {
+    BatchDesc &D = b->descs[i];
+    const BatchForm form = unit_count[i] ? batch_form(D) : kBatchEbSr;
+    BatchPart &own = b->parts[split && form != kBatchEbSr ? 1 : 0];
+    for (auto &p : b->parts) p.prefix[i + 1] = p.prefix[i];
+    D.unit_begin = own.prefix[i];
+    own.prefix[i + 1] += unit_count[i];
+    own.lds = std::max(own.lds, item_lds[i]);
+    own.form = std::max(own.form, form);
+  }
 
   auto fail = [&](hipError_t e, const char *what) {
     const int32_t s = hip_error(e, what);
@@ -259,23 +290,26 @@ int32_t segtaco_batch_create(const segtaco_batch_item_t *items, int32_t n,
   }
   const size_t nd = sizeof(BatchDesc) * (size_t)(n > 0 ? n : 1);
   if ((e = hipMalloc(&b->d_desc, nd)) != hipSuccess) return fail(e, "hipMalloc(descs)");
-  if ((e = hipMalloc(&b->d_prefix, sizeof(int64_t) * (n + 1))) != hipSuccess)
+  if ((e = hipMalloc(&b->d_prefix, sizeof(int64_t) * (n + 1) * kParts)) != hipSuccess)
     return fail(e, "hipMalloc(prefix)");
   if ((e = hipMalloc(&b->d_fix_prefix, sizeof(int64_t) * (n + 1))) != hipSuccess)
     return fail(e, "hipMalloc(fix prefix)");
-  if ((e = hipMalloc(&b->d_counter, sizeof(unsigned long long))) != hipSuccess)
+  if ((e = hipMalloc(&b->d_counter, kCounterStride * kParts)) != hipSuccess)
     return fail(e, "hipMalloc(counter)");
   if (n > 0 && (e = hipMemcpy(b->d_desc, b->descs.data(), sizeof(BatchDesc) * n,
                               hipMemcpyHostToDevice)) != hipSuccess)
     return fail(e, "hipMemcpy(descs)");
-  if ((e = hipMemcpy(b->d_prefix, b->prefix.data(), sizeof(int64_t) * (n + 1),
-                     hipMemcpyHostToDevice)) != hipSuccess)
-    return fail(e, "hipMemcpy(prefix)");
+  for (int p = 0; p < kParts; ++p)
+    if ((e = hipMemcpy(b->d_prefix + (size_t)p * (n + 1), b->parts[p].prefix.data(),
+                       sizeof(int64_t) * (n + 1), hipMemcpyHostToDevice)) != hipSuccess)
+      return fail(e, "hipMemcpy(prefix)");
   if ((e = hipMemcpy(b->d_fix_prefix, b->fix_prefix.data(), sizeof(int64_t) * (n + 1),
                      hipMemcpyHostToDevice)) != hipSuccess)
     return fail(e, "hipMemcpy(fix prefix)");
-  if ((e = batch_main_grid(b_dtype, b->lds, &b->grid, b->form)) != hipSuccess)
-    return fail(e, "batch_main_grid");
+  for (auto &p : b->parts)
+    if (p.units() > 0 &&
+        (e = batch_main_grid(b_dtype, p.lds, &p.grid, p.form)) != hipSuccess)
+      return fail(e, "batch_main_grid");
   if ((e = hipStreamSynchronize(stream)) != hipSuccess) return fail(e, "hipStreamSynchronize");
   *out = b;
   return SEGTACO_OK;
@@ -285,9 +319,15 @@ int32_t segtaco_batch_run(segtaco_batch_t b, void *stream_v) {
   if (!b) return set_error(SEGTACO_ERR_INVALID, "null batch");
   hipStream_t s = static_cast<hipStream_t>(stream_v);
   if (b->n == 0) return SEGTACO_OK;
-  SEGTACO_HIP(launch_batch_main(b->dt, b->d_desc, b->n, b->d_prefix, b->total_units,
-                                b->d_counter, b->grid, b->lds, s, /*reset_counter=*/true,
-                                b->form));
+  SEGTACO_HIP(launch_batch_reset(b->d_counter, kCounterStride, kParts, s));
+  for (int p = 0; p < kParts; ++p) {
+    const BatchPart &q = b->parts[p];
+    if (q.units() == 0) continue;
+    SEGTACO_HIP(launch_batch_main(
+        b->dt, b->d_desc, b->n, b->d_prefix + (size_t)p * (b->n + 1), q.units(),
+        reinterpret_cast<unsigned long long *>(b->d_counter + p * kCounterStride), q.grid,
+        q.lds, s, q.form));
+  }
   SEGTACO_HIP(launch_batch_fixup(b->d_desc, b->n, b->d_fix_prefix, b->total_fix, s));
   return SEGTACO_OK;
 }
@@ -342,7 +382,9 @@ int32_t segtaco_batch_partition(segtaco_batch_t b, int32_t i, int32_t *ntiles,
   return SEGTACO_OK;
 }
 
-int64_t segtaco_batch_units(segtaco_batch_t b) { return b ? b->total_units : -1; }
+int64_t segtaco_batch_units(segtaco_batch_t b) {
+  return b ? b->parts[0].units() + b->parts[1].units() : -1;
+}
 
 size_t segtaco_batch_workspace_bytes(segtaco_batch_t b) {
   return b ? b->ws_bytes : 0;

@@ -6,7 +6,9 @@
 
 namespace segtaco {
 
-__global__ void k_batch_reset(unsigned long long *counter) { *counter = 0ull; }
+__global__ void k_batch_reset(char *counters, size_t stride) {
+  *reinterpret_cast<unsigned long long *>(counters + threadIdx.x * stride) = 0ull;
+}
 
 __global__ __launch_bounds__(kBlockThreads) void k_batch_fixup(
     const BatchDesc *__restrict__ d, int32_t n,
@@ -49,13 +51,16 @@ hipError_t batch_main_grid(int dt, size_t lds, int32_t *grid, BatchForm form) {
 #undef RUN
 }
 
+hipError_t launch_batch_reset(char *counters, size_t stride, int32_t count, hipStream_t s) {
+  hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3((unsigned)count), 0, s, counters, stride);
+  return hipGetLastError();
+}
+
 hipError_t launch_batch_main(int dt, const BatchDesc *d, int32_t n,
                              const int64_t *prefix, int64_t total,
                              unsigned long long *counter, int32_t grid,
-                             size_t lds, hipStream_t s, bool reset_counter, BatchForm form) {
-  if (reset_counter) hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(1), 0, s, counter);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || total <= 0) return e;
+                             size_t lds, hipStream_t s, BatchForm form) {
+  if (total <= 0) return hipSuccess;
 #define RUN(DT, F) return launch_batch_main_t<DT, F>(d, n, prefix, total, counter, grid, lds, s)
   SEGTACO_BATCH_DISPATCH(RUN)
 #undef RUN

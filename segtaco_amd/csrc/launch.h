@@ -103,16 +103,16 @@ struct BatchDesc {
 enum BatchForm : int32_t { kBatchEbSr = 0, kBatchAny = 1, kBatchSv = 2 };
 
 // Persistent launch over `total` units (prefix[i] = first unit of product i,
-// non-decreasing, n entries); workgroups take units from *counter, which the
-// launcher resets first with a one-thread kernel unless reset_counter is
-// false (the caller has already put a zero there on the same stream).
-// grid = persistent workgroups (batch_main_grid), lds = dynamic LDS; form: the
-// largest batch_form of the products, which selects the kernel.
+// non-decreasing, n entries); workgroups take units from *counter, which holds
+// zero when the launch starts (launch_batch_reset, or copied there on the same
+// stream). grid = persistent workgroups (batch_main_grid), lds = dynamic LDS; form:
+// the largest batch_form of the products with units, which selects the kernel.
 hipError_t launch_batch_main(int dt, const BatchDesc *d, int32_t n,
                              const int64_t *prefix, int64_t total,
                              unsigned long long *counter, int32_t grid,
-                             size_t lds, hipStream_t s, bool reset_counter = true,
-                             BatchForm form = kBatchAny);
+                             size_t lds, hipStream_t s, BatchForm form);
+// Zeroes `count` 64-bit counters, `stride` bytes apart.
+hipError_t launch_batch_reset(char *counters, size_t stride, int32_t count, hipStream_t s);
 hipError_t launch_batch_fixup(const BatchDesc *d, int32_t n,
                               const int64_t *fix_prefix, int64_t total,
                               hipStream_t s);
@@ -125,6 +125,6 @@ void fill_batch_desc(const segtaco_csr_t &A, const void *B, int64_t ldb,
                      const segtaco_plan_t &plan, BatchDesc *D, int64_t *units,
                      int64_t *fix_units, size_t *lds, EbLayout *lay);
 // Workgroups of the persistent launch that fit the device at once.
-hipError_t batch_main_grid(int dt, size_t lds, int32_t *grid, BatchForm form = kBatchAny);
+hipError_t batch_main_grid(int dt, size_t lds, int32_t *grid, BatchForm form);
 
 }  // namespace segtaco

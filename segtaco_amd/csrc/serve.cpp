@@ -486,8 +486,7 @@ void launch_tick(segtaco_server *s, int32_t si) {
                        hipMemcpyHostToDevice, slot.stream);
   if (e == hipSuccess && n > 0)
     e = launch_batch_main(s->cfg.dtype, slot.d_desc, n, slot.d_prefix, total,
-                          slot.d_counter, grid, lds, slot.stream, /*reset_counter=*/false,
-                          form);
+                          slot.d_counter, grid, lds, slot.stream, form);
   if (e == hipSuccess && n > 0)
     e = launch_batch_fixup(slot.d_desc, n, slot.d_fix, total_fix, slot.stream);
   if (e == hipSuccess) e = hipEventRecord(slot.done, slot.stream);
