@@ -61,6 +61,8 @@ hipError_t launch_batch_main(int dt, const BatchDesc *d, int32_t n,
                              unsigned long long *counter, int32_t grid,
                              size_t lds, hipStream_t s, BatchForm form) {
   if (total <= 0) return hipSuccess;
+  // workgroups without a unit would only queue at the counter (5 ns each)
+  if (grid > total) grid = (int32_t)total;
 #define RUN(DT, F) return launch_batch_main_t<DT, F>(d, n, prefix, total, counter, grid, lds, s)
   SEGTACO_BATCH_DISPATCH(RUN)
 #undef RUN
