@@ -1,9 +1,11 @@
 """Which kernel form a plan runs with, and sizing for plans whose fields no
 call would accept (host logic, no GPU)."""
+import math
 import os
 import subprocess
 import sys
 
+import numpy as np
 import pytest
 
 import segtaco_amd as S
@@ -108,3 +110,26 @@ def test_segment_form_by_size(dtype, tile, N, nnz, seg):
     assert _form(N, dtype, nnz=nnz, M=2 * nnz + 1, tile=tile)["seg_vec"] == 0
     if N % 2 == 0:
         assert _form(N, dtype, nnz=nnz, tile=tile, vec=1)["seg_vec"] == 0
+
+
+# Plans that were measured with kernels of another generation are not taken from a
+# saved cache: the signature they were saved under is no matrix's any more.
+def test_old_cache_entries_do_not_match():
+
+    def signature(st, N, dtype, salt):
+        h = 1469598103934665603
+        near = lambda x: int(math.floor(x + 0.5))
+        for v in (st.M.bit_length() - 1, near(math.log2(st.mean_len) * 4), near(st.cv * 4),
+                  near(st.frac_nnz_long * 10), (st.max_len + 1).bit_length() - 1, N, dtype, salt):
+            for b in (v & (2 ** 64 - 1)).to_bytes(8, "little"):
+                h = ((h ^ b) * 1099511628211) & (2 ** 64 - 1)
+        return h
+
+    st = S.row_stats(np.cumsum([0] + [3, 9, 27, 1] * 500).astype(np.int32), 4000)
+    for N in (16, 64, 128):
+        assert S.tune_signature(st, N) == signature(st, N, S.DT_F32, 8)
+        S.tune_cache_clear()
+        S.tune_cache_put(signature(st, N, S.DT_F32, 7), S.make_plan("rb_pr", vec=1, col_lanes=4,
+                                                                    group=16, comp_threshold=0))
+        assert S.tune(st, N).as_dict() == S.tune_model(st, N).as_dict()
+    S.tune_cache_clear()
