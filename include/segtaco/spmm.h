@@ -221,7 +221,10 @@ typedef struct segtaco_plan {
                              all that a row can use, up to 64 (rb_pr 16,
                              eb_pr 32); rb_sr and eb_sr keep another value */
   int32_t group;          /* *_pr: nnz slots reduced together (power of two);
-                             rb_sr: rows per lane group; 0 = auto */
+                             rb_sr: rows per lane group, 1..16, kept in the
+                             plan but without effect: a launch runs one row
+                             per lane group, more of them in flight, which
+                             measured faster than 2; 0 = auto */
   int32_t tile;           /* eb_*: nnz per tile (multiple of 8); 0 = auto:
                              eb_sr 128, halved (down to 8) while the product
                              would fill fewer than two workgroups per compute
@@ -326,7 +329,7 @@ int32_t segtaco_block_starts(const int32_t *pos, int32_t M,
 /* ------------------------------------------------------------------------ */
 /* Partition introspection: the row partitions the schedules run on          */
 /* ------------------------------------------------------------------------ */
-#define SEGTACO_ROWS_SCATTER 0 /* one pass over pos (standalone calls, SDDMM) */
+#define SEGTACO_ROWS_SCATTER 0 /* one pass over pos (standalone calls) */
 #define SEGTACO_ROWS_SEARCH 1  /* K21 search + repair per tile (batches, server) */
 
 /* rows[b] = the row holding stored entry b*tile for b < ntiles =

@@ -4,8 +4,7 @@
 // the cost that dominates):
 //   * near-uniform row lengths (max <= 4 x mean and cv < 0.6, e.g. banded
 //     or fixed-degree matrices): rb_sr — one lane group per row, sequential
-//     sums, no partition or fix-up pass; short rows get several rows per
-//     lane group so a workgroup still carries ~1K entries;
+//     sums, no partition or fix-up pass;
 //   * skewed (power-law) lengths: eb_sr — equal-entry tiles keep every lane
 //     group equally busy whatever the tail; tile 128 for short mean rows,
 //     256 above 32 entries per row.
@@ -63,10 +62,12 @@ bool shared_schedule(int32_t sched) {
   return sched >= SEGTACO_RB_SR && sched <= SEGTACO_EB_PR;
 }
 
-bool same_plan(const segtaco_plan_t &a, const segtaco_plan_t &b) {
-  return a.schedule == b.schedule && a.vec == b.vec &&
-         a.col_lanes == b.col_lanes && a.group == b.group &&
-         a.tile == b.tile && a.comp_threshold == b.comp_threshold;
+// Plans that launch the same (rb_sr runs one row per lane group whatever its
+// group says).
+bool same_launch(const segtaco_plan_t &a, const segtaco_plan_t &b) {
+  return a.schedule == b.schedule && a.vec == b.vec && a.col_lanes == b.col_lanes &&
+         (a.group == b.group || a.schedule == SEGTACO_RB_SR) && a.tile == b.tile &&
+         a.comp_threshold == b.comp_threshold;
 }
 
 segtaco_csr_t shape_only(const segtaco_row_stats_t *st, int32_t dt) {
@@ -92,7 +93,8 @@ int32_t tune_model_impl(const segtaco_row_stats_t *st, int32_t N,
     p.schedule = SEGTACO_RB_SR;
     p.group = 1;
     SEGTACO_RET(plan_resolve_impl(&A, N, b_dtype, N, N, &p));
-    // Rows per lane group so that one workgroup walks ~1K entries.
+    // Rows per lane group so that one workgroup walks ~1K entries: what the plan
+    // says, though the launch runs one.
     const double rows_per_block = (double)kWavesPerBlock * (64 / p.col_lanes);
     int32_t g = 1;
     while (g < 16 && rows_per_block * g * (mean > 0.5 ? mean : 0.5) < 1024.0) g <<= 1;
@@ -244,7 +246,6 @@ int32_t segtaco_tune_measure(const segtaco_csr_t *A,
   std::vector<segtaco_plan_t> cands = {
       model,
       make(SEGTACO_RB_SR, 0, 0, 0, 0),
-      make(SEGTACO_RB_SR, 0, 0, 4, 0),
       make(SEGTACO_RB_PR, 0, 0, 0, 0),
       make(SEGTACO_RB_PR, 0, 0, 8, 0),
       make(SEGTACO_EB_SR, 0, 0, 0, 64),
@@ -259,7 +260,7 @@ int32_t segtaco_tune_measure(const segtaco_csr_t *A,
   for (auto p : cands) {
     if (plan_resolve_impl(A, N, b_dtype, ldb, ldc, &p) != SEGTACO_OK) continue;
     bool dup = false;
-    for (const auto &q : plans) dup = dup || same_plan(p, q);
+    for (const auto &q : plans) dup = dup || same_launch(p, q);
     if (dup) continue;
     plans.push_back(p);
     const size_t w = spmm_workspace_bytes_impl(A, N, &p);

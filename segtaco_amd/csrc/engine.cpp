@@ -625,9 +625,9 @@ int32_t spmm_impl(const segtaco_csr_t *A, const void *B, int32_t b_dtype,
                                   (phases & kPhaseWalk) != 0);
   const int32_t V = form.vec;
   a.lq = form.lq;
-  // rb_sr's rows per group only order the launch: one row per group keeps
-  // more rows in flight (uniform 100003 x 90001, 20 entries per row, N = 32
-  // FP32: 42 -> 36 us against two rows, BF16 30 -> 22)
+  // rb_sr's rows per group would only order the launch, and one row per group
+  // keeps more rows in flight (uniform 100003 x 90001, 20 entries per row, N = 32
+  // FP32: 42 -> 36 us against two rows, BF16 30 -> 22): the plan's is not used
   a.lg = plan.schedule == SEGTACO_RB_SR ? 0 : ilog2(plan.group);
   a.tile = plan.tile;
   a.comp_threshold = plan.comp_threshold == 0 ? INT_MAX : plan.comp_threshold;

@@ -11,7 +11,9 @@
 //   spmm_eb_pr_<Nnz>_<gs> (spmm_eb_pr.h:482-779): Nnz entries per tile ->
 //     tile = Nnz; gs lanes per segmented reduction -> group = gs slots.
 //   spmm_rb_sr_256_<r>_<c> (spmm_rb_sr.h:351-535): r rows per thread ->
-//     group = r rows per lane group; c columns per thread -> vec cap c.
+//     group = r rows per lane group (in the plan only: every launch runs one row
+//     per lane group, so presets that differ in r alone run the same kernel);
+//     c columns per thread -> vec cap c.
 //   spmm_eb_sr_256_<g>_<c> (spmm_eb_sr.h:856-1095): g entries per group of a
 //     64*g*c-entry block -> tile = 64*g entries per lane group; c columns per
 //     thread -> vec cap c.
