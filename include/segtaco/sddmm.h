@@ -10,7 +10,8 @@
  * stores S's values, X and Y as FP32, BF16 or FP16 and accumulates in FP32;
  * each entry's dot product has a fixed order (per-lane sequential over V
  * elements, then a butterfly over the lanes), so results are deterministic.
- * It reuses the SpMM path's row partition (the repaired K21 array).
+ * Each wave finds the rows of its entries itself (those of the repaired K21
+ * array).
  */
 #ifndef SEGTACO_SDDMM_H
 #define SEGTACO_SDDMM_H
@@ -23,7 +24,8 @@
 extern "C" {
 #endif
 
-/* Device bytes of workspace segtaco_sddmm needs for S. */
+/* Device bytes of workspace segtaco_sddmm asks for with S. The present kernel
+ * leaves it untouched; the call still refuses a smaller one. */
 size_t segtaco_sddmm_workspace_bytes(const segtaco_csr_t *S);
 
 /* out[p] for p < S->nnz (device pointers; asynchronous on `stream`). X is

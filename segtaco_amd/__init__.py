@@ -684,7 +684,7 @@ ROWS_SEARCH = 1
 def tile_rows(pos_ptr: int, M: int, T: int, ntiles: int, rows_ptr: int, method: int,
               part_ptr: int | None = None, stream: int | None = None) -> None:
     """First row of every element-balanced tile (K21 search + repair), on
-    device; method ROWS_SCATTER (standalone calls, SDDMM) or ROWS_SEARCH
+    device; method ROWS_SCATTER (standalone calls) or ROWS_SEARCH
     (batches, server; also the K21 array into part_ptr)."""
     check(lib().segtaco_tile_rows(pos_ptr, M, T, ntiles, method, rows_ptr, part_ptr or None,
                                   stream or None))

@@ -219,13 +219,6 @@ __device__ __forceinline__ void load_lds(const T *p, T (&x)[n]) {
   __builtin_memcpy(x, __builtin_assume_aligned(p, 16), sizeof(x));
 }
 
-template <int DT, int V, bool kOff32>
-__device__ __forceinline__ void load_row_vec(const void *__restrict__ base,
-                                             int32_t row, int64_t ld, int32_t c,
-                                             float (&out)[V]) {
-  unpack<DT, V>(load_row_raw<DT, V, kOff32>(base, row, ld, c), out);
-}
-
 // Makes this wave's LDS writes visible to all of its lanes: a release/acquire
 // fence at wavefront scope around a wave barrier (no block-wide s_barrier).
 __device__ __forceinline__ void wave_sync() {
