@@ -157,8 +157,11 @@ __device__ __forceinline__ void rb_sr_row(const KArgs &a, int32_t row, int32_t p
 // The sum of the n > 0 entries p, p + 2^lg, ... of a slot of rb_pr. A batch loads
 // no entries that are not there: where B stays in the caches the loads themselves
 // are the time (banded, 33 entries per row, 8 slots, us per call, all four loads /
-// those needed: FP32 N = 4 21 / 16, N = 64 176 / 159, BF16 N = 1 18 / 14).
-template <int DT, int V, bool kOff32, bool kComp>
+// those needed: FP32 N = 4 21 / 16, N = 64 176 / 159, BF16 N = 1 18 / 14). kAll: all
+// four all the same, for the four-set form, whose time is its longest row's chain of
+// batches (power-law 60013 x 50021, FP32 N = 4: 21.7 us, 23.3 with the tests in the
+// chain); chosen per wave, the two loops' registers cost the banded calls their gain.
+template <int DT, int V, bool kOff32, bool kComp, bool kAll>
 __device__ __forceinline__ void rb_pr_sum(const KArgs &a, int32_t p, int32_t n, int lg,
                                           int32_t col, float (&acc)[V]) {
   using R = typename RawT<DT, V>::type;
@@ -166,11 +169,12 @@ __device__ __forceinline__ void rb_pr_sum(const KArgs &a, int32_t p, int32_t n, 
   float cmp[V], v[U];
   zero_vec(cmp);
   int32_t c[U];
+  const int32_t last = p + ((n - 1) << lg);
   auto entries = [&](int32_t b) {
-    if (b + U <= n) {
+    if (kAll || b + U <= n) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const int32_t i = p + ((b + u) << lg);
+        const int32_t i = !kAll || b + u < n ? p + ((b + u) << lg) : last;
         c[u] = a.crd[i];
         v[u] = load_val<DT>(a.vals, i);
       }
@@ -202,7 +206,7 @@ __device__ __forceinline__ void rb_pr_sum(const KArgs &a, int32_t p, int32_t n, 
   if (b < n) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (b + u < n) x[u] = load_row_raw<DT, V, kOff32>(a.B, c[u], a.ldb, col);
+      if (kAll || b + u < n) x[u] = load_row_raw<DT, V, kOff32>(a.B, c[u], a.ldb, col);
 #pragma unroll
     for (int u = 0; u < U; ++u) rb_add_if<DT, V, kComp>(b + u < n, x[u], v[u], acc, cmp);
   }
@@ -312,16 +316,16 @@ __device__ __forceinline__ void rb_pr_walk(const KArgs &a, int32_t blk,
     for (int k = 0; k < R; ++k) {
       if (n[k] > 0 && comp[k]) {
         zero_vec(acc[k]);
-        rb_pr_sum<DT, V, kOff32, true>(a, p[k], n[k], lg, col, acc[k]);
+        rb_pr_sum<DT, V, kOff32, true, (R > 1)>(a, p[k], n[k], lg, col, acc[k]);
       } else if (n[k] > 1) {
-        rb_pr_sum<DT, V, kOff32, false>(a, p[k] + P, n[k] - 1, lg, col, acc[k]);
+        rb_pr_sum<DT, V, kOff32, false, (R > 1)>(a, p[k] + P, n[k] - 1, lg, col, acc[k]);
       }
     }
   } else if (n[0] > 0) {
     if (comp[0])
-      rb_pr_sum<DT, V, kOff32, true>(a, p[0], n[0], lg, col, acc[0]);
+      rb_pr_sum<DT, V, kOff32, true, (R > 1)>(a, p[0], n[0], lg, col, acc[0]);
     else
-      rb_pr_sum<DT, V, kOff32, false>(a, p[0], n[0], lg, col, acc[0]);
+      rb_pr_sum<DT, V, kOff32, false, (R > 1)>(a, p[0], n[0], lg, col, acc[0]);
   }
   // butterfly over the P slots of each row (lane distances Q*P/2 .. Q)
 #pragma unroll
