@@ -329,7 +329,8 @@ int32_t cs_vec(const segtaco_plan_t &p, int32_t N, int32_t b_dtype) {
 }  // namespace
 
 // The vector width and lanes a resolved plan runs with; no choice here changes
-// a sum's order.
+// a sum's order, but for eb_cs where a row's columns are not ascending: wider slots
+// are fewer, and which tiles sweep (column order) or walk (CSR order) goes by them.
 //
 // A plan that names a narrower slice than the operands allow, or for eb_sr and
 // rb_sr other lanes than the row spreads over, runs as it says. The rest is

@@ -10,7 +10,8 @@
 // different steps; a small one leaves most of the chip without a tile; and
 // both pay three launches (partition, walk, fix-up).
 //
-// Here a wave takes a range of whole tiles (128 to 384 entries):
+// Here a wave takes a range of whole tiles, one at least: up to 384 entries (128 at
+// N = 16), less where that would leave fewer than 2048 waves, a longer tile alone:
 //   * it finds the range's rows itself (a 64-way search of pos, three
 //     dependent loads for 262144 rows), so there is no partition launch;
 //   * all lanes gather the range's B slices, entry after entry, whatever row
@@ -34,7 +35,10 @@
 // entries, 26 of the 66 us); the 4.2 M gathers, one 128-byte line each, need
 // about 12 us. Ranges of 128 to 1024 entries measured within 30 % of the best
 // at each width: longer ones balance the groups, shorter ones let more waves
-// share a CU's LDS.
+// share a CU's LDS. Tiles shorter than a range cost its piece lists and the later
+// pieces' sums (60000^2, N = 4: 24 at tile 128, 35 at tile 8), and the 16 gathers per
+// lane are more than a short range fills: at N <= 4, where a wave's 64 groups cover
+// 1024 entries, ten of them re-load the last of 384.
 #include "device_common.h"
 #include "seg.h"
 

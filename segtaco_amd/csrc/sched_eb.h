@@ -65,7 +65,7 @@ constexpr int kPrPasses = 8;       // eb_pr passes whose gathers are in flight
 // eb_sr chunk: the LDS per block stays under 64 KiB for every lane count, and a
 // short tile takes no more than its entries, since the LDS of a batch's largest
 // product decides how many workgroups all of them have (32 products, one of
-// them 4 lanes and tile 16, BF16: 4.3 ms per launch with 64-entry chunks, 3.5 so).
+// them 4 lanes and tile 16, BF16: 4.3 ms per launch with 64-entry chunks, 3.3 so).
 __host__ __device__ inline int32_t eb_sr_chunk(int32_t lq, int32_t tile) {
   const int32_t c = 16 << lq;
   const int32_t whole = tile < kSrChunkMax ? (tile + 15) & ~15 : kSrChunkMax;
