@@ -157,6 +157,10 @@ void fill_batch_desc(const segtaco_csr_t &A, const void *B, int64_t ldb,
     }
   }
   *units = (int64_t)a.nblocks * a.panels;
+  if (A.nnz == 0) {  // zeros alone: the fix-up writes them, in rb_sr's units
+    *fix_units = *units;
+    *units = 0;
+  }
 }
 
 }  // namespace segtaco

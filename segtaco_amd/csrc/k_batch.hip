@@ -3,11 +3,20 @@
 // batched carry fix-up.
 #include "batch_main.h"
 #include "sched_eb.h"
+#include "sched_rb.h"
 
 namespace segtaco {
 
 __global__ void k_batch_reset(char *counters, size_t stride) {
   *reinterpret_cast<unsigned long long *>(counters + threadIdx.x * stride) = 0ull;
+}
+
+template <int V>
+__device__ __forceinline__ void fixup_unit(const KArgs &a, int32_t blk, int32_t panel) {
+  if (a.nnz == 0)
+    zero_rows<V>(a, blk, panel);
+  else
+    fixup_body<V>(a, blk, panel);
 }
 
 __global__ __launch_bounds__(kBlockThreads) void k_batch_fixup(
@@ -21,10 +30,10 @@ __global__ __launch_bounds__(kBlockThreads) void k_batch_fixup(
     const int32_t panel = (int32_t)(local % a.panels);
     const int32_t blk = (int32_t)(local / a.panels);
     switch (D.vec) {
-      case 1: fixup_body<1>(a, blk, panel); break;
-      case 2: fixup_body<2>(a, blk, panel); break;
-      case 4: fixup_body<4>(a, blk, panel); break;
-      default: fixup_body<8>(a, blk, panel); break;
+      case 1: fixup_unit<1>(a, blk, panel); break;
+      case 2: fixup_unit<2>(a, blk, panel); break;
+      case 4: fixup_unit<4>(a, blk, panel); break;
+      default: fixup_unit<8>(a, blk, panel); break;
     }
   }
 }

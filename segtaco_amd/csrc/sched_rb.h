@@ -216,6 +216,20 @@ __device__ __forceinline__ void rb_pr_sum(const KArgs &a, int32_t p, int32_t n, 
   }
 }
 
+// Zeros to the rows of rb_sr's row block `blk`, column panel `panel`.
+template <int V>
+__device__ __forceinline__ void zero_rows(const KArgs &a, int32_t blk, int32_t panel) {
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int64_t row =
+      ((int64_t)(blk * kWavesPerBlock + wave) << (6 - a.lq)) + (lane >> a.lq);
+  const int32_t nominal = ((panel << a.lq) + (lane & ((1 << a.lq) - 1))) * V;
+  float z[V];
+  zero_vec(z);
+  if (row < a.M && nominal < a.N)
+    store_row<V>(a.C + row * a.ldc + lane_col<V>(nominal, a.N), z);
+}
+
 // rb_sr over row block `blk`, column panel `panel`: lane group gi owns row gi.
 template <int DT, int V, bool kLean, bool kOff32>
 __device__ __forceinline__ void rb_sr_walk(const KArgs &a, int32_t blk,

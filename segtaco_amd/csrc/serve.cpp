@@ -463,7 +463,7 @@ void launch_tick(segtaco_server *s, int32_t si) {
     slot.h_prefix[i + 1] = total;
     slot.h_fix[i + 1] = total_fix;
     lds = std::max(lds, l);
-    form = std::max(form, batch_form(D));
+    if (units) form = std::max(form, batch_form(D));
     r.flops = 2.0 * m.nnz * r.N;
   }
   const int32_t n = (int32_t)chosen.size();
