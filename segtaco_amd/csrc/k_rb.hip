@@ -1,5 +1,6 @@
 // k_rb.hip — standalone launches of the row-balanced schedules (bodies in
 // sched_rb.h): one workgroup per (row block, column panel).
+#include "engine.h"
 #include "sched_rb.h"
 
 namespace segtaco {
@@ -19,10 +20,17 @@ __global__ __launch_bounds__(kBlockThreads) void k_rb_pr(const KArgs a) {
 }
 
 template <int DT, int V>
+__global__ __launch_bounds__(kBlockThreads) void k_rb_pr_all(const KArgs a) {
+  int32_t blk, panel;
+  if (!decode_block(a.panels, a.nblocks, blk, panel)) return;
+  rb_pr_body<DT, V, 1, true>(a, blk, panel);
+}
+
+template <int DT, int V>
 __global__ __launch_bounds__(kBlockThreads) void k_rb_pr4(const KArgs a) {
   int32_t blk, panel;
   if (!decode_block(a.panels, a.nblocks, blk, panel)) return;
-  rb_pr_body<DT, V, 4>(a, blk, panel);
+  rb_pr_body<DT, V, 4, true>(a, blk, panel);
 }
 
 #define SEGTACO_CASE(KERNEL, DT, V, grid, args, stream)                        \
@@ -70,6 +78,10 @@ hipError_t launch_rb_pr(int dt, int vec, const KArgs &a, hipStream_t s) {
   // 20.7 / 16.1; 262144^2 N = 1 64 / 41; but even rows of 20 entries at N = 16
   // (P = 16) 33 / 44, and 16-byte slices of 16-bit B lose to their registers
   // (262144^2 BF16 N = 16 128 / 147).
+  if (grid <= 4 * (int64_t)device_cus()) {
+    SEGTACO_DISPATCH(k_rb_pr_all, dt, vec, grid, a, s);
+    return hipGetLastError();
+  }
   if (grid < 8192 || vec == 8 || a.nnz > (int64_t)a.M << a.lg) {
     SEGTACO_DISPATCH(k_rb_pr, dt, vec, grid, a, s);
     return hipGetLastError();

@@ -158,9 +158,11 @@ __device__ __forceinline__ void rb_sr_row(const KArgs &a, int32_t row, int32_t p
 // no entries that are not there: where B stays in the caches the loads themselves
 // are the time (banded, 33 entries per row, 8 slots, us per call, all four loads /
 // those needed: FP32 N = 4 21 / 16, N = 64 176 / 159, BF16 N = 1 18 / 14). kAll: all
-// four all the same, for the four-set form, whose time is its longest row's chain of
-// batches (power-law 60013 x 50021, FP32 N = 4: 21.7 us, 23.3 with the tests in the
-// chain); chosen per wave, the two loops' registers cost the banded calls their gain.
+// four all the same, for launches whose time is their longest row's chain of
+// batches, which the tests would lengthen: the four-set form (power-law 60013 x
+// 50021, FP32 N = 4: 21.7 us, 23.3 with the tests) and launches of up to four
+// workgroups per CU (power-law 20000^2, FP32 N = 4, 8 slots: 23 and 26 us). Chosen per
+// wave, the two loops' registers cost the banded calls their gain.
 template <int DT, int V, bool kOff32, bool kComp, bool kAll>
 __device__ __forceinline__ void rb_pr_sum(const KArgs &a, int32_t p, int32_t n, int lg,
                                           int32_t col, float (&acc)[V]) {
@@ -269,7 +271,7 @@ __device__ __forceinline__ void rb_sr_body(const KArgs &a, int32_t blk,
 // longer rows one set after another, and adjacent rows are often alike (lengths
 // in rising order, 100000^2, us per call, a wave's sets adjacent / so: FP32 N = 3
 // 65 / 57, N = 8 69 / 63, BF16 N = 12 163 / 135; one set per wave 47, 44, 131).
-template <int DT, int V, bool kOff32, int R>
+template <int DT, int V, bool kOff32, int R, bool kAll>
 __device__ __forceinline__ void rb_pr_walk(const KArgs &a, int32_t blk,
                                            int32_t panel) {
   const int lane = threadIdx.x & 63;
@@ -330,16 +332,16 @@ __device__ __forceinline__ void rb_pr_walk(const KArgs &a, int32_t blk,
     for (int k = 0; k < R; ++k) {
       if (n[k] > 0 && comp[k]) {
         zero_vec(acc[k]);
-        rb_pr_sum<DT, V, kOff32, true, (R > 1)>(a, p[k], n[k], lg, col, acc[k]);
+        rb_pr_sum<DT, V, kOff32, true, kAll>(a, p[k], n[k], lg, col, acc[k]);
       } else if (n[k] > 1) {
-        rb_pr_sum<DT, V, kOff32, false, (R > 1)>(a, p[k] + P, n[k] - 1, lg, col, acc[k]);
+        rb_pr_sum<DT, V, kOff32, false, kAll>(a, p[k] + P, n[k] - 1, lg, col, acc[k]);
       }
     }
   } else if (n[0] > 0) {
     if (comp[0])
-      rb_pr_sum<DT, V, kOff32, true, (R > 1)>(a, p[0], n[0], lg, col, acc[0]);
+      rb_pr_sum<DT, V, kOff32, true, kAll>(a, p[0], n[0], lg, col, acc[0]);
     else
-      rb_pr_sum<DT, V, kOff32, false, (R > 1)>(a, p[0], n[0], lg, col, acc[0]);
+      rb_pr_sum<DT, V, kOff32, false, kAll>(a, p[0], n[0], lg, col, acc[0]);
   }
   // butterfly over the P slots of each row (lane distances Q*P/2 .. Q)
 #pragma unroll
@@ -351,13 +353,13 @@ __device__ __forceinline__ void rb_pr_walk(const KArgs &a, int32_t blk,
   }
 }
 
-template <int DT, int V, int R = 1>
+template <int DT, int V, int R = 1, bool kAll = false>
 __device__ __forceinline__ void rb_pr_body(const KArgs &a, int32_t blk,
                                            int32_t panel) {
   if (a.b_off32)
-    rb_pr_walk<DT, V, true, R>(a, blk, panel);
+    rb_pr_walk<DT, V, true, R, kAll>(a, blk, panel);
   else
-    rb_pr_walk<DT, V, false, R>(a, blk, panel);
+    rb_pr_walk<DT, V, false, R, kAll>(a, blk, panel);
 }
 
 }  // namespace segtaco
