@@ -54,6 +54,7 @@ struct segtaco_batch {
   BatchPart parts[kParts];
   std::vector<int64_t> fix_prefix;
   int64_t total_fix = 0;
+  int64_t zero_units = 0;  // of products without entries, in the fix-up
   BatchDesc *d_desc = nullptr;
   int64_t *d_prefix = nullptr, *d_fix_prefix = nullptr;  // d_prefix: per part, n + 1
   char *d_counter = nullptr;
@@ -243,6 +244,7 @@ int32_t segtaco_batch_create(const segtaco_batch_item_t *items, int32_t n,
     fill_batch_desc(A, it.B, it.ldb, it.C, it.ldc, it.N, b_dtype, plan, &D, &units,
                     &fix_units, &lds, &lay[i]);
     unit_count[i] = units;
+    if (A.nnz == 0) b->zero_units += fix_units;
     item_lds[i] = lds;
     if (batch_form(D) == kBatchEbSr && D.vec < 4) narrow += A.nnz;
     if (plan.schedule >= SEGTACO_EB_SR) {
@@ -387,7 +389,7 @@ int32_t segtaco_batch_partition(segtaco_batch_t b, int32_t i, int32_t *ntiles,
 }
 
 int64_t segtaco_batch_units(segtaco_batch_t b) {
-  return b ? b->parts[0].units() + b->parts[1].units() : -1;
+  return b ? b->parts[0].units() + b->parts[1].units() + b->zero_units : -1;
 }
 
 size_t segtaco_batch_workspace_bytes(segtaco_batch_t b) {

@@ -54,6 +54,11 @@ def test_parts_have_the_bits_of_single_calls(dtype):
         if A.nnz and (id(A), n, p.schedule) not in want:
             want[id(A), n, p.schedule] = run_spmm(A, Bd, n, p, b_dtype=dtype)
     batch = S.Batch(items, dtype, stream_ptr())
+    alone = [S.Batch([i], dtype, stream_ptr()) for i in items]
+    assert all(a.units() > 0 for a in alone)
+    assert batch.units() == sum(a.units() for a in alone)
+    for a in alone:
+        a.destroy()
     batch.capture()
     for step in range(4):
         for o in outs:
